@@ -439,6 +439,12 @@ int mcdp_debug_reverse_tiles(mcdp_propagator *prop, int64_t max_tiles);
  * step, every event a wave per group of 64 samples).  Results do not depend on
  * the route; tests use it to run both. */
 int mcdp_debug_tail_mode(mcdp_propagator *prop, int32_t mode);
+/* 1 if a run of n samples (injected: mcdp_propagate_*, otherwise mcdp_run_many_*
+ * with a durations output) takes the two-pass route of short runs -- every
+ * duration first, then the propagation level by level -- instead of a partial
+ * round of the walk.  Results do not depend on it, and a shape set by
+ * mcdp_propagator_configure or a tail mode rules it out. */
+int mcdp_debug_short_run(mcdp_propagator *prop, int32_t injected, int64_t n, int32_t *two_pass);
 /* The serving footprint rule, host only: for a request of n samples over a
  * context of n_events events and n_preds predecessor entries (at most
  * max_entries for one event: up to 254, chunks store one-byte winner

@@ -63,7 +63,7 @@ int mcdp_batch_create(mcdp_propagator *const *props, int32_t n_props, int32_t wa
     if (samples_per_lane != 1 && samples_per_lane != 2)
         return fail(MCDP_E_INVALID, "samples_per_lane must be 1 or 2");
     for (int32_t i = 0; i < n_props; ++i) {  // one schedule shape for every plan of the launch
-        int rc = configure_shape(props[i], waves, events_per_wave, samples_per_lane);
+        int rc = configure_shape(props[i], waves, events_per_wave, samples_per_lane, false);
         if (rc) return rc;
     }
     auto *b = new (std::nothrow) mcdp_batch;

@@ -309,6 +309,9 @@ constexpr size_t kLdsBudgetBytes = 64 * 1024;  // LDS per workgroup for predeces
 // Sample indices and leading dimensions are 32-bit in the kernel; tiles of up
 // to 128 samples must not overflow them.
 constexpr int64_t kMaxSamplesPerLaunch = ((int64_t)1 << 31) - 256;
+// The two-pass route of short runs is considered up to this many samples
+// (a round of tiles is 32,768 on 256 CUs).
+constexpr int64_t kLevelMaxSamples = (int64_t)1 << 17;
 
 // A predecessor record for edge l: its minimal duration, sampling kind and p0
 // inline; the distribution index for the kinds that read more parameters.
@@ -332,6 +335,18 @@ Record edge_record(const mcdp_propagator &P, int32_t l) {
     return r;
 }
 
+// Relative cost of evaluating event e for one wave.
+int event_cost(const mcdp_propagator &P, int32_t e) {
+    int c = kEventCost;
+    for (int64_t k = P.pred_off[(size_t)e]; k < P.pred_off[(size_t)e + 1]; ++k) {
+        const int32_t l = P.preds[(size_t)k].edge;
+        const DistRec *D =
+            (l >= 0 && l < P.L && P.ldist[(size_t)l] != kNoDistIndex) ? &P.dist[P.ldist[(size_t)l]] : nullptr;
+        c += kPredCost + draw_cost(D);
+    }
+    return c;
+}
+
 // Steps, wave assignment, LDS slots and record streams for W waves per
 // workgroup and at most K events per wave and step.
 int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
@@ -349,16 +364,6 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
     P.tile_cost = 0;
     P.wide_cost = 0;
 
-    auto event_cost = [&](int32_t e) {
-        int c = kEventCost;
-        for (int64_t k = P.pred_off[(size_t)e]; k < P.pred_off[(size_t)e + 1]; ++k) {
-            const int32_t l = P.preds[(size_t)k].edge;
-            const DistRec *D = (l >= 0 && l < L && P.ldist[(size_t)l] != kNoDistIndex) ? &P.dist[P.ldist[(size_t)l]] : nullptr;
-            c += kPredCost + draw_cost(D);
-        }
-        return c;
-    };
-
     // (a) steps: each level in as few steps as W x K events allow, split evenly;
     // within a step, events go to the least-loaded wave (longest first).
     std::vector<int32_t> ev_step((size_t)E, -1);
@@ -371,7 +376,7 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
         for (size_t c = 0; c < nsteps; ++c) {
             const size_t c0 = lev.size() * c / nsteps, c1 = lev.size() * (c + 1) / nsteps;
             std::vector<std::pair<int, int32_t>> items;
-            for (size_t i = c0; i < c1; ++i) items.emplace_back(event_cost(lev[i]), lev[i]);
+            for (size_t i = c0; i < c1; ++i) items.emplace_back(event_cost(P, lev[i]), lev[i]);
             std::stable_sort(items.begin(), items.end(), [](auto &a, auto &b) { return a.first > b.first; });
             std::vector<std::vector<int32_t>> per((size_t)W);
             std::vector<int64_t> load((size_t)W, 0);
@@ -477,7 +482,7 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
         for (int32_t w = 0; w < W; ++w) {
             int64_t c = 0;
             for (int32_t i = P.ev_off[(size_t)t * W + w]; i < P.ev_off[(size_t)t * W + w + 1]; ++i) {
-                const int64_t ce = event_cost(flat_events[(size_t)i]);
+                const int64_t ce = event_cost(P, flat_events[(size_t)i]);
                 c += ce;
                 costliest = std::max(costliest, ce);
             }
@@ -489,6 +494,65 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
     for (int32_t l = 0; l < L; ++l)
         if (!referenced[(size_t)l]) P.orph.push_back(edge_record(P, l));
     return MCDP_OK;
+}
+
+// LDS slots of the two-pass route: an event that a later level reads has one
+// from its own level to the last that reads it.  level_kernel writes a level's
+// results while other waves may still read for that level, so a slot is given
+// out again from the level after its last read.
+void build_level_slots(mcdp_propagator &P) {
+    const int32_t n_levels = (int32_t)P.levels.size();
+    std::vector<int32_t> level((size_t)P.E, 0), last_use((size_t)P.E, -1);
+    P.level_width = 0;
+    P.walk_cost = 0;
+    for (int32_t t = 0; t < n_levels; ++t) {
+        P.level_width = std::max<int32_t>(P.level_width, (int32_t)P.levels[(size_t)t].size());
+        int64_t sum = 0, costliest = 0;
+        for (int32_t e : P.levels[(size_t)t]) {
+            level[(size_t)e] = t;
+            const int64_t c = event_cost(P, e);
+            sum += c;
+            costliest = std::max(costliest, c);
+        }
+        P.walk_cost += std::max(costliest, (sum + kMaxWaves - 1) / kMaxWaves);
+    }
+    for (int32_t e = 0; e < P.E; ++e)
+        for (int64_t k = P.pred_off[(size_t)e]; k < P.pred_off[(size_t)e + 1]; ++k) {
+            const PredEntry &pe = P.preds[(size_t)k];
+            if (!pe.stale) last_use[(size_t)pe.src] = std::max(last_use[(size_t)pe.src], level[(size_t)e]);
+        }
+    P.level_slot.assign((size_t)P.E, -1);
+    std::vector<std::vector<int32_t>> release((size_t)n_levels + 1);
+    std::vector<int32_t> free_slots;
+    // slot 0 holds NaN; each event that is read stale has one for its earliest time
+    int32_t used = 1;
+    P.level_stale.clear();
+    P.level_zero_edges = false;
+    for (const PredEntry &pe : P.preds) {
+        if (pe.stale) P.level_stale.emplace_back(pe.src, 0);
+        P.level_zero_edges |= pe.edge < 0 || pe.edge >= P.L;
+    }
+    std::sort(P.level_stale.begin(), P.level_stale.end());
+    P.level_stale.erase(std::unique(P.level_stale.begin(), P.level_stale.end()), P.level_stale.end());
+    for (auto &st : P.level_stale) st.second = used++;
+    for (int32_t t = 0; t < n_levels; ++t) {
+        for (int32_t slot : release[(size_t)t]) free_slots.push_back(slot);
+        for (int32_t e : P.levels[(size_t)t]) {
+            if (last_use[(size_t)e] < 0) continue;
+            int32_t slot;
+            if (free_slots.empty()) {
+                slot = used++;
+            } else {
+                slot = free_slots.back();
+                free_slots.pop_back();
+            }
+            P.level_slot[(size_t)e] = slot;
+            release[(size_t)last_use[(size_t)e] + 1].push_back(slot);
+        }
+    }
+    P.level_slots = used;
+    // the plan packs slots and predecessor counts into 15 and 16 bits
+    if (used > 0x7FFF || max_entries(P) > 0xFFFF) P.level_slots = std::numeric_limits<int32_t>::max();
 }
 
 // Default (waves, events per wave) for a DAG: enough waves to spread the widest
@@ -630,6 +694,7 @@ int compile_propagator(mcdp_propagator &P, int32_t n_events, const double *earli
     P.E = E;
     P.L = L;
     P.earliest.assign(earliest, earliest + E);
+    build_level_slots(P);
 
     // (6) default schedule.
     int32_t W, K;
@@ -637,18 +702,145 @@ int compile_propagator(mcdp_propagator &P, int32_t n_events, const double *earli
     return build_schedule(P, W, K);
 }
 
-// Uploads the plan of `P` to the current device (once per device).
-int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
+// The two-pass route's plan with P's current times: every event in level
+// order with its predecessors, and a record per link, costliest laws first
+// (waves of draw_kernel take them in turn, so the last ones are short).
+struct LevelPlan {
+    std::vector<int32_t> off, extra_of;
+    std::vector<LevelQuad> quad;
+    std::vector<LevelPred> extra;
+    std::vector<LevelInit> init;
+    std::vector<Record> draws;
+};
+LevelPlan level_plan(const mcdp_propagator &P) {
+    LevelPlan lv;
+    const size_t E = (size_t)P.E;
+    lv.init.push_back(LevelInit{std::numeric_limits<double>::quiet_NaN(), 0, 0});
+    for (const auto &st : P.level_stale) lv.init.push_back(LevelInit{P.earliest[(size_t)st.first], st.second, 0});
+    auto entry = [&](const PredEntry &pe) {
+        LevelPred pr{0, pe.edge >= 0 && pe.edge < P.L ? pe.edge : -1, pe.src};
+        pr.slot = !pe.stale ? P.level_slot[(size_t)pe.src]
+                            : std::lower_bound(P.level_stale.begin(), P.level_stale.end(), std::make_pair(pe.src, 0))->second;
+        return pr;
+    };
+    auto pair16 = [](int32_t lo, int32_t hi) { return (int32_t)((uint32_t)(lo & 0xFFFF) | (uint32_t)hi << 16); };
+    lv.quad.resize(E * kLevelQuads);
+    lv.extra_of.assign(E, 0);
+    lv.off.assign(1, 0);
+    size_t q = 0;
+    for (const auto &level : P.levels) {
+        for (int32_t e : level) {
+            const int64_t p0 = P.pred_off[(size_t)e], p1 = P.pred_off[(size_t)e + 1];
+            const double times[2] = {P.earliest[(size_t)e], P.earliest[(size_t)e] + P.max_delay};
+            std::memcpy(&lv.quad[q], times, sizeof(times));
+            LevelPred pr[kLevelPreds];
+            for (int k = 0; k < kLevelPreds; ++k)
+                pr[k] = p0 + k < p1 ? entry(P.preds[(size_t)(p0 + k)]) : LevelPred{0, k ? pr[0].edge : 0, -1};
+            lv.extra_of[(size_t)e] = (int32_t)lv.extra.size();
+            for (int64_t k = p0 + kLevelPreds; k < p1; ++k) lv.extra.push_back(entry(P.preds[(size_t)k]));
+            lv.quad[E + q] = LevelQuad{{e, pair16(P.level_slot[(size_t)e], (int32_t)(p1 - p0)),
+                                        pair16(pr[0].slot, pr[1].slot), pair16(pr[2].slot, pr[3].slot)}};
+            lv.quad[2 * E + q] = LevelQuad{{pr[0].edge, pr[1].edge, pr[2].edge, pr[3].edge}};
+            lv.quad[3 * E + q] = LevelQuad{{pr[0].src, pr[1].src, pr[2].src, pr[3].src}};
+            ++q;
+        }
+        lv.off.push_back((int32_t)q);
+    }
+    lv.off.push_back((int32_t)q);
+    std::vector<std::pair<int, int32_t>> order((size_t)P.L);
+    for (int32_t l = 0; l < P.L; ++l) {
+        const uint32_t di = P.ldist[(size_t)l];
+        // by cost, equal costs by law: a wave's links then mostly share theirs
+        const int cost = di == kNoDistIndex ? draw_cost(nullptr) : draw_cost(&P.dist[di]);
+        order[(size_t)l] = {-(cost * 64 + (di == kNoDistIndex ? 0 : (int)(P.dist[di].kind & 63))), l};
+    }
+    std::stable_sort(order.begin(), order.end(), [](auto &a, auto &b) { return a.first < b.first; });
+    lv.draws.reserve((size_t)P.L);
+    for (auto &o : order) lv.draws.push_back(edge_record(P, o.second));
+    return lv;
+}
+
+// P's entry for the current device.
+int device_entry_impl(mcdp_propagator &P, DeviceCopy *&out) {
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
         return fail(MCDP_E_DEVICE, "no HIP device available: the Monte Carlo engine runs on the GPU only");
     int device = 0;
     HIP_TRY(hipGetDevice(&device), "hipGetDevice");
+    out = nullptr;
     for (auto &d : P.dev)
-        if (d.device == device) {
-            out = &d;
-            return MCDP_OK;
+        if (d.device == device) out = &d;
+    if (!out) {
+        P.dev.push_back(DeviceCopy{});
+        out = &P.dev.back();
+        out->device = device;
+    }
+    return MCDP_OK;
+}
+
+// Device allocation for the parts added to it, and their upload.
+class Upload {
+   public:
+    template <typename T>
+    size_t add(const std::vector<T> &v) {
+        const size_t o = host_.size();
+        host_.resize(o + align_up(std::max<size_t>(v.size() * sizeof(T), 1), 256));
+        if (!v.empty()) std::memcpy(host_.data() + o, v.data(), v.size() * sizeof(T));
+        return o;
+    }
+    int send(void *&blob) {
+        blob = nullptr;
+        hipError_t e = hipMalloc(&blob, std::max<size_t>(host_.size(), 256));
+        if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
+        e = hipMemcpy(blob, host_.data(), host_.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(blob);
+            blob = nullptr;
+            return hip_fail(e, "hipMemcpy (plan)");
         }
+        return MCDP_OK;
+    }
+
+   private:
+    std::vector<unsigned char> host_;
+};
+template <typename T>
+const T *part(const void *blob, size_t offset) {
+    return reinterpret_cast<const T *>(static_cast<const unsigned char *>(blob) + offset);
+}
+
+// Uploads the two-pass route's plan to d's device (once).
+int ensure_levels(const mcdp_propagator &P, DeviceCopy &d) {
+    if (d.level_blob) return MCDP_OK;
+    const LevelPlan lv = level_plan(P);
+    Upload up;
+    const size_t o_off = up.add(lv.off), o_quad = up.add(lv.quad), o_xof = up.add(lv.extra_of), o_init = up.add(lv.init),
+                 o_extra = up.add(lv.extra), o_draws = up.add(lv.draws), o_dist = up.add(P.dist),
+                 o_alias = up.add(P.alias);
+    const int rc = up.send(d.level_blob);
+    if (rc) return rc;
+    const void *b = d.level_blob;
+    d.levels.off = part<int32_t>(b, o_off);
+    d.levels.quad = part<LevelQuad>(b, o_quad);
+    d.levels.extra_of = part<int32_t>(b, o_xof);
+    d.levels.init = part<LevelInit>(b, o_init);
+    d.levels.n_init = (int32_t)lv.init.size();
+    d.levels.extra = part<LevelPred>(b, o_extra);
+    d.levels.E = P.E;
+    d.levels.n_levels = (int32_t)P.levels.size();
+    d.draws.recs = part<Record>(b, o_draws);
+    d.draws.dists = part<DistParams>(b, o_dist);
+    d.draws.alias = part<AliasRec>(b, o_alias);
+    d.draws.n_alias = (int32_t)P.alias.size();
+    d.draws.L = P.L;
+    return MCDP_OK;
+}
+
+// Uploads the walk's plan of `P` to the current device (once per device).
+int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
+    const int rc = device_entry_impl(P, out);
+    if (rc || out->blob) return rc;
+    DeviceCopy &d = *out;
     const size_t a = 256;
     size_t off = 0;
     auto reserve = [&](size_t bytes) {
@@ -694,9 +886,6 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
         (void)hipFree(blob);
         return hip_fail(e, "hipMemcpy (plan)");
     }
-    DeviceCopy d;
-    d.device = device;
-    d.blob = blob;
     // the side stream of wide steps and its fork / join events, made here so
     // that a launch creates nothing (it may be under stream capture)
     e = hipStreamCreateWithFlags(&d.side, hipStreamNonBlocking);
@@ -705,9 +894,12 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
     if (e != hipSuccess) {
         if (d.side) (void)hipStreamDestroy(d.side);
         if (d.fork) (void)hipEventDestroy(d.fork);
+        d.side = nullptr;
+        d.fork = nullptr;
         (void)hipFree(blob);
         return hip_fail(e, "side stream");
     }
+    d.blob = blob;
     auto *b = static_cast<unsigned char *>(blob);
     d.base.step_off = reinterpret_cast<const int32_t *>(b + o_step);
     d.base.recs = reinterpret_cast<const Record *>(b + o_recs);
@@ -724,8 +916,6 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
     d.base.waves = P.waves;
     d.base.n_alias = (int32_t)P.alias.size();
     d.base.slots = P.slots;
-    P.dev.push_back(d);
-    out = &P.dev.back();
     return MCDP_OK;
 }
 // The fast kernel variant needs every read predecessor in LDS (or stale) and
@@ -812,10 +1002,77 @@ int choose_shape(mcdp_propagator &P) {
     return build_schedule(P, best.waves, best.k);
 }
 
+// Samples per workgroup of level_kernel for a run of n: the fewest that leave
+// no more workgroups than CUs (a workgroup costs a level's latency whatever it
+// carries, and a second one per CU waits for the first), within what LDS
+// holds; 0 if the DAG keeps more realized times live than LDS holds for one
+// sample.  Measured on the network DAG, propagation alone: 4,001 samples 0.77 ms
+// at 16 a workgroup against 0.86 at 8 and 1.28 at 32; 1,000 samples 0.26 ms at 4
+// against 0.38 at 2 and 0.34 at 8.
+int level_group(const mcdp_propagator &P, int64_t n, int cus) {
+    int group = 1;
+    while (group < kLevelMaxGroup && (n + group - 1) / group > cus) group *= 2;
+    while (group > 0 && (size_t)P.level_slots * (size_t)group * sizeof(double) > kLevelLdsMaxBytes) group /= 2;
+    return group;
+}
+
+// Whether a run of n samples takes the two-pass route (draw_kernel, then
+// level_kernel) instead of a partial round of the walk: when its estimated time
+// is below a tile's.  The walk's tile costs the same however few of its lanes
+// and of the device's CUs are in use: 12 ns per unit of walk_cost (200 x 100
+// events, any n up to a round: 3.3 ms; 20 x 10: 93 us).  The two passes move
+// the durations twice, at about 3.9 TB/s where they are bound by that, but at
+// least a level's latency per level (200 x 100, sampled: 1 sample 0.11 ms, 4,001
+// 1.20, 8,192 2.25 against 2.3 with wide steps, 12,345 3.9 against 3.3; 60 x 250:
+// 12,345 3.3 against 4.8).
+constexpr double kTileSecondsPerCost = 12e-9;
+constexpr double kLevelSeconds = 0.45e-6;       // one level of one workgroup
+constexpr double kLevelFixedSeconds = 10e-6;    // the second launch, the tables
+constexpr double kLevelBytesPerSecond = 3.9e12;
+bool level_route(const mcdp_propagator &P, bool injected, int64_t n, int cus) {
+    if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
+    const int group = level_group(P, n, cus);
+    if (group == 0) return false;
+    const double per_pass = (double)group * cus;  // samples of one workgroup per CU
+    const double padded = std::ceil((double)n / per_pass) * per_pass;
+    const double draws = injected ? 0.0 : (double)n * 8.0 * P.L / kLevelBytesPerSecond;
+    const double moved = (n > per_pass ? padded : (double)n) * (8.0 * P.L + 12.0 * P.E) / kLevelBytesPerSecond;
+    const double waves = (n > per_pass ? padded / per_pass : 1.0);
+    const double levels = std::max(moved, waves * kLevelSeconds * (double)P.levels.size());
+    return kLevelFixedSeconds + draws + levels < kTileSecondsPerCost * (double)P.walk_cost;
+}
+
+int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injected, const int32_t *seeds,
+                       const double *dur_in, int64_t n, int64_t ld, double *realized, double *durations,
+                       int32_t *cause, uint8_t *cause_pos, int cus, hipStream_t stream) {
+    if (!injected) {
+        DrawParams q = d.draws;
+        q.seeds = seeds;
+        q.n = (int32_t)n;
+        q.ld = (int32_t)ld;
+        q.durations = durations;
+        HIP_TRY(launch_draws(q, cus, stream), "draw kernel launch");
+    }
+    LevelParams p = d.levels;
+    p.dur = injected ? dur_in : durations;
+    p.n = (int32_t)n;
+    p.ld = (int32_t)ld;
+    p.realized = realized;
+    p.cause = cause;
+    p.cause_pos = cause_pos;
+    const int group = level_group(P, n, cus);
+    const int64_t want = (int64_t)P.level_width * group;
+    const int threads = (int)std::min<int64_t>((want + kLanes - 1) / kLanes * kLanes, kLevelMaxThreads);
+    HIP_TRY(launch_levels(p, P.level_zero_edges, group, threads, P.level_slots, stream), "level kernel launch");
+    return MCDP_OK;
+}
+
 // cause_pos (sampled walks, no cause): the winning entry's position per
-// sample instead of the cause event.
+// sample instead of the cause event.  scratch: [L][ld] or null, for a sampled
+// run without a durations output that may take the two-pass route.
 int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double *dur_in, int64_t n, int64_t ld,
-           double *realized, double *durations, int32_t *cause, hipStream_t stream, uint8_t *cause_pos = nullptr) {
+           double *realized, double *durations, int32_t *cause, hipStream_t stream, uint8_t *cause_pos = nullptr,
+           double *scratch = nullptr) {
     if (n < 0) return fail(MCDP_E_INVALID, "n must be non-negative");
     if (cause_pos && (injected || cause)) return fail(MCDP_E_INVALID, "internal error: positions replace sampled causes");
     if (n > 0 && ld < n) return fail(MCDP_E_INVALID, "ld must be >= n");
@@ -825,16 +1082,31 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     if (!injected && !seeds && n > 0) return fail(MCDP_E_INVALID, "seeds is null");
     if (!realized && P.E > 0 && n > 0) return fail(MCDP_E_INVALID, "realized must not be null");
     std::lock_guard<std::mutex> lock(P.mu);
-    int count = 0;
-    if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
-        return fail(MCDP_E_DEVICE, "no HIP device available: the Monte Carlo engine runs on the GPU only");
-    if (!P.shape_fixed) {  // first launch: fit the schedule to this device
-        int rc = choose_shape(P);
+    DeviceCopy *d = nullptr;
+    int rc = device_entry_impl(P, d);
+    if (rc) return rc;
+    int cus = 0, bpc = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d->device), "hipDeviceGetAttribute");
+    // A short run takes the two-pass route where there is room for its
+    // durations.  Its plan is uploaded by the first such run: one under
+    // stream capture, which can upload nothing, walks unless it is there.
+    double *const drawn = durations ? durations : scratch;
+    if (n > 0 && (injected || drawn) && level_route(P, injected, n, cus)) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (!d->level_blob) (void)hipStreamIsCapturing(stream, &capture);
+        if (capture == hipStreamCaptureStatusNone) {
+            rc = ensure_levels(P, *d);
+            return rc ? rc
+                      : launch_level_route(P, *d, injected, seeds, dur_in, n, ld, realized, drawn, cause, cause_pos, cus,
+                                           stream);
+        }
+    }
+    if (!P.shape_fixed) {  // first walk: fit the schedule to this device
+        rc = choose_shape(P);
         if (rc) return rc;
         P.shape_fixed = true;
     }
-    DeviceCopy *d = nullptr;
-    int rc = ensure_device_impl(P, d);
+    rc = ensure_device_impl(P, d);
     if (rc) return rc;
     if (n == 0 || (P.E == 0 && (injected || P.orph.empty()))) return MCDP_OK;
     WalkParams p = d->base;
@@ -848,8 +1120,6 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     WalkVariant v = walk_variant(P, injected);
     v.pos = cause_pos != nullptr;
     const size_t lds = walk_lds_bytes(P, v);
-    int cus = 0, bpc = 0;
-    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d->device), "hipDeviceGetAttribute");
     HIP_TRY(walk_occupancy(v, P.waves, lds, &bpc), "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     if (bpc < 1) return fail(MCDP_E_DEVICE, "walk kernel cannot be resident with " + std::to_string(lds) + " bytes of LDS");
     const int64_t resident = (int64_t)cus * bpc;
@@ -1217,6 +1487,10 @@ int launch_host_chunk(mcdp_propagator &P, HostWork *hw, bool injected, const int
         return launch(P, injected, d_seeds, d_dur, m, ld, d_real, injected ? nullptr : d_dur, d_cause, st);
     };
     if (!hw || m != ld || m > kGraphMaxSamples || P.n_steps < kGraphMinSteps) return direct();
+    bool two_pass = false;  // two launches: no graph
+    const int qc = short_run(P, injected, m, two_pass);
+    if (qc) return qc;
+    if (two_pass) return direct();
     ShortRunKey key;
     key.buf = hw->buf;
     key.n = m;
@@ -1382,6 +1656,17 @@ int run_host(mcdp_propagator &P, bool injected, const int32_t *seeds, const doub
 
 }  // namespace
 
+int mcdp::device_entry(mcdp_propagator &P, DeviceCopy *&out) { return device_entry_impl(P, out); }
+
+int mcdp::short_run(mcdp_propagator &P, bool injected, int64_t n, bool &yes) {
+    std::lock_guard<std::mutex> lock(P.mu);
+    int device = 0, cus = 0;
+    HIP_TRY(hipGetDevice(&device), "hipGetDevice");
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device), "hipDeviceGetAttribute");
+    yes = n > 0 && level_route(P, injected, n, cus);
+    return MCDP_OK;
+}
+
 int mcdp::ensure_device(mcdp_propagator &P, DeviceCopy *&out) {
     // The uploaded plan must be the one the walk kernel will run: fix the
     // schedule shape first, as the first launch would.
@@ -1397,9 +1682,6 @@ int mcdp::ensure_device(mcdp_propagator &P, DeviceCopy *&out) {
 }
 mcdp::WalkVariant mcdp::plan_variant(const mcdp_propagator &P, bool injected) { return walk_variant(P, injected); }
 size_t mcdp::plan_lds_bytes(const mcdp_propagator &P, WalkVariant v) { return walk_lds_bytes(P, v); }
-int mcdp::configure_shape(mcdp_propagator *prop, int32_t waves, int32_t k, int32_t spl) {
-    return mcdp_propagator_configure(prop, waves, k, spl);
-}
 mcdp::Record mcdp::link_record(const mcdp_propagator &P, int32_t l) { return edge_record(P, l); }
 
 int32_t mcdp::max_entries(const mcdp_propagator &P) {
@@ -1409,12 +1691,12 @@ int32_t mcdp::max_entries(const mcdp_propagator &P) {
 }
 
 int mcdp::run_many_positions(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
-                             uint8_t *cause_pos, hipStream_t s) {
+                             uint8_t *cause_pos, hipStream_t s, double *scratch) {
     if (!cause_pos) return fail(MCDP_E_INVALID, "positions output is null");
     if (max_entries(P) > kMaxPositionEntries)
         return fail(MCDP_E_INVALID, "winner positions need events of at most 254 predecessor entries");
     if (n > 0 && !seeds_dev) return fail(MCDP_E_INVALID, "seeds is null");
-    return launch(P, false, seeds_dev, nullptr, n, ld, realized, nullptr, nullptr, s, cause_pos);
+    return launch(P, false, seeds_dev, nullptr, n, ld, realized, nullptr, nullptr, s, cause_pos, scratch);
 }
 
 // The range of every duration the sampler can draw for link l, as the device
@@ -1686,8 +1968,10 @@ int mcdp_propagator_ranges(const mcdp_propagator *prop, double *link_lo, double 
     return MCDP_OK;
 }
 
-int mcdp_propagator_configure(mcdp_propagator *prop, int32_t waves, int32_t events_per_wave,
-                              int32_t samples_per_lane) {
+}  // extern "C"
+
+int mcdp::configure_shape(mcdp_propagator *prop, int32_t waves, int32_t events_per_wave, int32_t samples_per_lane,
+                          bool by_caller) {
     if (!prop) return fail(MCDP_E_INVALID, "propagator is null");
     if (!shape_valid(waves, events_per_wave, samples_per_lane))
         return fail(MCDP_E_INVALID,
@@ -1699,7 +1983,15 @@ int mcdp_propagator_configure(mcdp_propagator *prop, int32_t waves, int32_t even
     prop->spl = samples_per_lane;
     prop->drop_device_copies();
     prop->shape_fixed = true;
+    prop->shape_by_caller = by_caller;
     return MCDP_OK;
+}
+
+extern "C" {
+
+int mcdp_propagator_configure(mcdp_propagator *prop, int32_t waves, int32_t events_per_wave,
+                              int32_t samples_per_lane) {
+    return configure_shape(prop, waves, events_per_wave, samples_per_lane, true);
 }
 
 int mcdp_propagator_autotune(mcdp_propagator *prop, int64_t n_samples, int32_t *waves, int32_t *events_per_wave,
@@ -1734,7 +2026,7 @@ int mcdp_propagator_autotune(mcdp_propagator *prop, int64_t n_samples, int32_t *
     if (e == hipSuccess) e = hipEventCreate(&t1);
     if (e != hipSuccess) rc = hip_fail(e, "autotune setup");
     for (size_t c = 0; rc == MCDP_OK && c < cands.size(); ++c) {
-        rc = mcdp_propagator_configure(prop, cands[c].waves, cands[c].k, cands[c].spl);
+        rc = configure_shape(prop, cands[c].waves, cands[c].k, cands[c].spl, true);  // time the walk, not the two passes
         if (rc) break;
         {  // skip shapes that cannot be resident
             std::lock_guard<std::mutex> lock(prop->mu);
@@ -1764,8 +2056,12 @@ int mcdp_propagator_autotune(mcdp_propagator *prop, int64_t n_samples, int32_t *
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
     (void)hipFree(buf);
-    if (rc) return rc;
-    rc = mcdp_propagator_configure(prop, best.waves, best.k, best.spl);
+    if (rc) {
+        std::lock_guard<std::mutex> lock(prop->mu);
+        prop->shape_by_caller = false;
+        return rc;
+    }
+    rc = configure_shape(prop, best.waves, best.k, best.spl, false);
     if (rc) return rc;
     if (waves) *waves = best.waves;
     if (events_per_wave) *events_per_wave = best.k;
@@ -1854,7 +2150,7 @@ int mcdp_propagator_autotune_cached(mcdp_propagator *prop, int64_t n_samples, co
         }
     }
     if (found) {
-        int rc = mcdp_propagator_configure(prop, got.waves, got.k, got.spl);
+        int rc = configure_shape(prop, got.waves, got.k, got.spl, false);
         if (rc) return rc;
         bool resident = false;
         {
@@ -1902,6 +2198,16 @@ int mcdp_debug_tail_mode(mcdp_propagator *prop, int32_t mode) {
     std::lock_guard<std::mutex> lock(prop->mu);
     prop->tail_mode = mode;
     return MCDP_OK;
+}
+
+int mcdp_debug_short_run(mcdp_propagator *prop, int32_t injected, int64_t n, int32_t *two_pass) {
+    if (!prop || !two_pass) return fail(MCDP_E_INVALID, "null argument");
+    int count = 0;
+    if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) return fail(MCDP_E_DEVICE, "no HIP device available");
+    bool yes = false;
+    const int rc = short_run(*prop, injected != 0, n, yes);
+    *two_pass = yes ? 1 : 0;
+    return rc;
 }
 
 // ---- device plumbing --------------------------------------------------------

@@ -35,11 +35,12 @@ int hip_fail(hipError_t e, const char *what);
 using DistRec = DistParams;
 constexpr uint32_t kNoDistIndex = 0xFFFFFFFFu;  // the link's type has no distribution
 
-// The plan (and, once statistics are asked for, the predecessor table) on one
-// device.
+// What of a propagator lives on one device: the walk's plan, the two-pass
+// route's, the statistics' predecessor table, the gradients' reverse plan;
+// each uploaded when it is first needed there.
 struct DeviceCopy {
     int device = -1;
-    void *blob = nullptr;
+    void *blob = nullptr;  // the walk's plan
     WalkParams base{};
     void *topo = nullptr;                // statistics: predecessor table, uploaded on first use
     const int32_t *pred_off = nullptr;   // [E + 1]
@@ -54,6 +55,9 @@ struct DeviceCopy {
     const Record *rev_unit_links = nullptr;
     void *rev_work = nullptr;            // partial rows and global slots
     size_t rev_work_bytes = 0;
+    void *level_blob = nullptr;          // short runs: the plan of the two-pass route
+    LevelParams levels{};
+    DrawParams draws{};
     // A second stream for the wide steps of a last partial round, which run
     // beside the tiles of the full rounds (created on first use), and the
     // events that fork it from and join it to the caller's stream.
@@ -148,6 +152,14 @@ struct mcdp_propagator {
     int32_t spl = 1;  // samples per lane of the walk kernel (schedule-independent)
     int64_t n_global = 0;
     bool shape_fixed = false;  // set by configure / autotune / the first launch
+    bool shape_by_caller = false;  // configure chose the walk's shape: short runs keep to the walk too
+    // the two-pass route of short runs (schedule-independent): LDS slot of
+    // each event (-1: no later level reads it), slots in all, widest level
+    std::vector<int32_t> level_slot;
+    std::vector<std::pair<int32_t, int32_t>> level_stale;  // (source, its slot), sources ascending
+    int32_t level_slots = 0, level_width = 0;
+    int64_t walk_cost = 0;  // a tile's walk in draw-cost units, by 16 waves evenly loaded
+    bool level_zero_edges = false;  // some predecessor's edge is outside the link table
     std::shared_ptr<mcdp::RevPlan> rev;  // built on the first gradient call
     int64_t rev_max_tiles = 0;           // test hook: tiles per reverse launch (0: default)
     // device copies, one per device used
@@ -170,6 +182,7 @@ struct mcdp_propagator {
             (void)hipSetDevice(d.device);
             (void)hipDeviceSynchronize();  // launches in flight on any stream may still read the plan
             if (d.blob) (void)hipFree(d.blob);
+            if (d.level_blob) (void)hipFree(d.level_blob);
             if (d.topo) (void)hipFree(d.topo);
             if (d.rev) (void)hipFree(d.rev);
             if (d.rev_work) (void)hipFree(d.rev_work);
@@ -199,6 +212,9 @@ namespace mcdp {
 // The propagator's plan on the current device (uploaded on first use).  The
 // caller holds P.mu.
 int ensure_device(mcdp_propagator &P, DeviceCopy *&out);
+// The propagator's entry for the current device, with or without its plans.
+// The caller holds P.mu.
+int device_entry(mcdp_propagator &P, DeviceCopy *&out);
 // Walk-kernel variant (fast or general paths) and its LDS bytes for P's plan.
 WalkVariant plan_variant(const mcdp_propagator &P, bool injected);
 size_t plan_lds_bytes(const mcdp_propagator &P, WalkVariant v);
@@ -219,8 +235,12 @@ int reverse_run(mcdp_propagator *prop, const int32_t *seeds_dev, const double *w
                 const double *durations_dev, const int32_t *cause_dev, int64_t n, int64_t ld, int accumulate,
                 double *objective_dev, double *grad_dmin_dev, double *grad_earliest_dev, void *work, size_t work_bytes,
                 hipStream_t s);
-// mcdp_propagator_configure.
-int configure_shape(mcdp_propagator *prop, int32_t waves, int32_t k, int32_t spl);
+// mcdp_propagator_configure (by_caller: short runs keep to the walk of that
+// shape, as its caller asked; otherwise they may take the two-pass route).
+int configure_shape(mcdp_propagator *prop, int32_t waves, int32_t k, int32_t spl, bool by_caller);
+// Whether a run of n samples takes the two-pass route where a durations buffer
+// is given (its results are the same bits).
+int short_run(mcdp_propagator &P, bool injected, int64_t n, bool &yes);
 // Uploads P's plan and the statistics' predecessor table to the current
 // device (what a resident context needs before serving requests).
 int prepare_stats(mcdp_propagator &P);
@@ -277,8 +297,9 @@ Record link_record(const mcdp_propagator &P, int32_t l);
 // asynchronous on s.
 constexpr int32_t kMaxPositionEntries = 254;
 int32_t max_entries(const mcdp_propagator &P);
+// scratch: [L][ld] or null, where short_run asks for it.
 int run_many_positions(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
-                       uint8_t *cause_pos, hipStream_t s);
+                       uint8_t *cause_pos, hipStream_t s, double *scratch = nullptr);
 // Bounds that hold for every seed: the durations link l can draw, and every
 // event's realized time (false when an earliest time or max_delay is not
 // finite).

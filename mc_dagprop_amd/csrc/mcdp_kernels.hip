@@ -388,6 +388,270 @@ __global__ void __launch_bounds__(kLanes) walk_wide_orphans_kernel(WalkParams p)
     p.durations[row_offset(rec.i2, (uint32_t)p.ld) + s] = dur[0];
 }
 
+// ---- short runs: all draws, then the propagation level by level -------------
+//
+// A run far smaller than a round of tiles leaves the fused walk waiting: one
+// tile walks the whole DAG on one CU, at a wave's own instruction latency.
+// Drawn first, the durations are independent of each other and fill the
+// device whatever the sample count; the propagation that is left is a few
+// instructions per predecessor.  Measured (one launch per step, or a tile,
+// before; two launches now), 200 x 100 events: 1 sample 1.34 -> 0.11 ms, 1,000
+// 1.09 -> 0.40, 4,001 1.77 -> 1.20; 60 x 250 events, 12,345 samples 4.8 -> 3.3;
+// 20 x 10 events, 1 sample 93 -> 17 us.
+
+// Every link's durations.  kLaneLinks: the lanes of a wave are 64 / group
+// links x group samples (short runs: the draw is divergent only where the
+// links' laws differ, and the records are sorted by law); otherwise a wave
+// takes kDrawSpl samples per lane of one link, its record in scalar registers.
+// A wave keeps its samples from link to link, so nothing but scalar loads and
+// table reads is waited for in its loop: a seed loaded there would wait for
+// the stores before it too.
+constexpr int kDrawBlock = 256;
+constexpr int kDrawSpl = 4;
+
+template <bool kLaneLinks>
+__global__ void __launch_bounds__(kDrawBlock) draw_kernel(DrawParams p, int32_t group, int32_t n_chunks,
+                                                          int32_t lds_alias_n) {
+    extern __shared__ double lds[];
+    __shared__ LogTableLds log_lds;
+    stage_log_table(log_lds);
+    AliasRec *const alias = reinterpret_cast<AliasRec *>(lds);
+    for (int i = threadIdx.x; i < lds_alias_n; i += kDrawBlock) alias[i] = p.alias[i];
+    __syncthreads();
+    const LogTable lt = log_lds.view();
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + (int)blockIdx.x * (kDrawBlock / kLanes);
+    const int waves = (int)gridDim.x * (kDrawBlock / kLanes);
+    const uint32_t ld = (uint32_t)p.ld;
+    const auto dists = as_const_space(p.dists);
+    if (kLaneLinks) {
+        // lanes past the last link or sample repeat the last one's draw and
+        // rewrite its bytes unchanged
+        const int32_t per = kLanes / group, sub = lane / group, sl = lane - sub * group;
+        const int32_t s = sl < p.n ? sl : p.n - 1;
+        const uint32_t seed[1] = {(uint32_t)p.seeds[s]};
+        for (int32_t l0 = wave * per; l0 < p.L; l0 += waves * per) {
+            const int32_t li = l0 + sub;
+            const Record r = p.recs[li < p.L ? li : p.L - 1];
+            double dur[1];
+            if (lds_alias_n > 0)
+                draw_durations<1>(r.info, r.a, r.b, (uint32_t)r.i2, seed, alias, dists, lt, dur);
+            else
+                draw_durations<1>(r.info, r.a, r.b, (uint32_t)r.i2, seed, as_const_space(p.alias), dists, lt, dur);
+            p.durations[row_offset(r.i2, ld) + s] = dur[0];
+        }
+    } else {
+        // waves chunk, chunk + n_chunks, ... share a chunk's links
+        const int32_t slices = waves / n_chunks;
+        const int32_t slice = wave / n_chunks, chunk = wave - slice * n_chunks;
+        if (slice >= slices) return;
+        int32_t s[kDrawSpl];
+        uint32_t seed[kDrawSpl];
+#pragma unroll
+        for (int i = 0; i < kDrawSpl; ++i) {
+            const int32_t si = chunk * (kLanes * kDrawSpl) + i * kLanes + lane;
+            s[i] = si < p.n ? si : p.n - 1;
+            seed[i] = (uint32_t)p.seeds[s[i]];
+        }
+        for (int32_t li = slice; li < p.L; li += slices) {
+            const Record r = as_const_space(p.recs)[li];
+            double dur[kDrawSpl];
+            if (lds_alias_n > 0)
+                draw_durations<kDrawSpl>(r.info, r.a, r.b, (uint32_t)r.i2, seed, alias, dists, lt, dur);
+            else
+                draw_durations<kDrawSpl>(r.info, r.a, r.b, (uint32_t)r.i2, seed, as_const_space(p.alias), dists, lt, dur);
+            double *const row = p.durations + row_offset(r.i2, ld);
+#pragma unroll
+            for (int i = 0; i < kDrawSpl; ++i) row[s[i]] = dur[i];
+        }
+    }
+}
+
+// The propagation: a workgroup carries `kGroup` samples through every level,
+// its threads being (item of the level, sample) pairs, the realized times that
+// later levels read in LDS slots.  A slot freed by a level's reads is given out
+// again from the next level on, so a level needs one barrier, after its
+// results are in their slots.  Nothing but the slots depends on an earlier
+// level: an item is loaded three steps ahead and its durations two steps
+// ahead, over the barriers, in a ring of four stages (the step is written out
+// once per position of the ring, so no stage is ever copied).  Bound by a
+// level's latency for few samples (0.45 us per level: loads one step ahead took
+// 1.0), by the durations' and results' bytes for many (16,384 samples of 200 x
+// 100 events: 10.5 GB in 2.7 ms, 3.9 TB/s, against 4.8 for a plain copy).
+struct LevelStage {
+    LevelQuad q[kLevelQuads];
+    double d[kLevelPreds];
+    bool valid, last;  // uniform: there is an item; it is in its level's last pass
+    bool live;         // this thread's item exists (a level's last pass may not fill the workgroup)
+};
+
+template <int kGroup, bool kZeroEdges>
+__global__ void __launch_bounds__(kLevelMaxThreads) level_kernel(LevelParams p) {
+    extern __shared__ double lds[];
+    const int sl = threadIdx.x & (kGroup - 1);
+    const int idx = threadIdx.x / kGroup;
+    const int stride = blockDim.x / kGroup;
+    // Workgroups go to the eight dies in turn: consecutive groups of samples
+    // share the cache lines of every row, so each die takes a run of them.
+    const int32_t per = ((int32_t)gridDim.x + 7) / 8;
+    const int32_t g = ((int32_t)blockIdx.x & 7) * per + ((int32_t)blockIdx.x >> 3);
+    const int32_t si = g * kGroup + sl;
+    if (g * kGroup >= p.n) return;  // the whole workgroup: g is uniform
+    const uint32_t s = (uint32_t)(si < p.n ? si : p.n - 1);
+    const uint32_t ld = (uint32_t)p.ld;
+    const auto off = as_const_space(p.off);
+    for (int i = idx; i < p.n_init; i += stride) lds[p.init[i].slot * kGroup + sl] = p.init[i].value;
+    __syncthreads();
+
+    // the next pass to fetch: items [q, q + stride) of the level ending at
+    // end.  Every fetch loads, past the last level its last item again, and
+    // every item loads a duration for each position, so that the number of
+    // loads is fixed and a wait for older ones leaves these in flight.
+    int32_t level = 0, q = off[0], end = off[1], end2 = off[2];
+    auto fetch = [&](LevelStage &x) {
+        x.valid = q < p.E;
+        const int32_t qi = q + idx;
+        x.live = qi < end;
+        const uint32_t byte = (uint32_t)(x.live ? qi : end - 1) * (uint32_t)sizeof(LevelQuad);
+#pragma unroll
+        for (int k = 0; k < kLevelQuads; ++k)
+            x.q[k] = *reinterpret_cast<const LevelQuad *>(reinterpret_cast<const char *>(p.quad + (int64_t)k * p.E) + byte);
+        q += stride;
+        x.last = q >= end;
+        if (x.last) {
+            q = end;
+            end = end2;
+            ++level;
+            end2 = off[level + 2 <= p.n_levels ? level + 2 : p.n_levels];
+        }
+    };
+    auto durations = [&](LevelStage &x) {
+#pragma unroll
+        for (int k = 0; k < kLevelPreds; ++k) {
+            const int32_t e = x.q[2].v[k];
+            x.d[k] = p.dur[row_offset(kZeroEdges && e < 0 ? 0 : e, ld) + s];
+        }
+    };
+    auto compute = [&](const LevelStage &x) {
+        const double upper = __hiloint2double(x.q[0].v[3], x.q[0].v[2]);
+        double best = __hiloint2double(x.q[0].v[1], x.q[0].v[0]);
+        int32_t who = -1;  // position of the winning predecessor
+        const int32_t event = x.q[1].v[0], slot = (int16_t)x.q[1].v[1], count = (uint32_t)x.q[1].v[1] >> 16;
+        auto take = [&](double rs, double d, int32_t k) {
+            double tt = rs + d;
+            tt = (upper < tt) ? upper : tt;
+            const bool wins = tt >= best;
+            best = wins ? tt : best;
+            who = wins ? k : who;
+        };
+        double rs[kLevelPreds];
+#pragma unroll
+        for (int k = 0; k < kLevelPreds; ++k) {
+            const uint32_t from = (k & 1) ? (uint32_t)x.q[1].v[2 + k / 2] >> 16 : (uint32_t)x.q[1].v[2 + k / 2] & 0xFFFFu;
+            rs[k] = lds[from * kGroup + sl];
+        }
+#pragma unroll
+        for (int k = 0; k < kLevelPreds; ++k) take(rs[k], kZeroEdges && x.q[2].v[k] < 0 ? 0.0 : x.d[k], k);
+        int32_t src = -1;
+        if (count > kLevelPreds) {
+            const int32_t first = p.extra_of[event];
+            for (int k = kLevelPreds; k < count; ++k) {
+                const LevelPred pr = p.extra[first + k - kLevelPreds];
+                double d = 0.0;
+                if (!kZeroEdges || pr.edge >= 0) d = p.dur[row_offset(pr.edge, ld) + s];
+                take(lds[pr.slot * kGroup + sl], d, k);
+                if (who == k) src = pr.src;
+            }
+        }
+        const double rr = (upper < best) ? upper : best;
+        if (x.live) {
+            if (slot >= 0) lds[slot * kGroup + sl] = rr;
+            const uint64_t row = row_offset(event, ld) + s;
+            p.realized[row] = rr;
+            if (p.cause_pos) {
+                p.cause_pos[row] = (uint8_t)who;
+            } else if (p.cause) {
+#pragma unroll
+                for (int k = 0; k < kLevelPreds; ++k) src = who == k ? x.q[3].v[k] : src;
+                p.cause[row] = src;
+            }
+        }
+    };
+    // one step of the ring: a computed, b's durations in flight, c's issued, d fetched
+    auto step = [&](LevelStage &a, LevelStage &b, LevelStage &c, LevelStage &d) {
+        fetch(d);
+        durations(c);
+        compute(a);
+        if (!b.valid) return false;
+        if (a.last) __syncthreads();
+        return true;
+    };
+    LevelStage a, b, c, d;
+    fetch(a);
+    fetch(b);
+    durations(a);
+    fetch(c);
+    durations(b);
+    while (step(a, b, c, d) && step(b, c, d, a) && step(c, d, a, b) && step(d, a, b, c)) {
+    }
+}
+
+hipError_t launch_draws(const DrawParams &p, int cus, hipStream_t stream) {
+    if (p.L <= 0 || p.n <= 0) return hipSuccess;
+    const size_t alias_bytes = (size_t)p.n_alias * sizeof(AliasRec);
+    const int32_t lds_alias_n = alias_bytes <= kAliasLdsMaxBytes ? p.n_alias : 0;
+    const size_t lds = lds_alias_n > 0 ? alias_bytes : 0;
+    constexpr int kWavesPerBlock = kDrawBlock / kLanes;
+    const int64_t most = (int64_t)cus * 8;  // blocks resident at once, about
+    if (p.n < kLanes) {
+        int32_t group = 1;
+        while (group < p.n) group *= 2;
+        const int64_t waves = ((int64_t)p.L * group + kLanes - 1) / kLanes;
+        const int64_t blocks = std::min<int64_t>((waves + kWavesPerBlock - 1) / kWavesPerBlock, most);
+        hipLaunchKernelGGL((draw_kernel<true>), dim3((unsigned)blocks), dim3(kDrawBlock), lds, stream, p, group, 0,
+                           lds_alias_n);
+    } else {
+        const int64_t chunks = ((int64_t)p.n + kLanes * kDrawSpl - 1) / (kLanes * kDrawSpl);
+        const int64_t need = (chunks + kWavesPerBlock - 1) / kWavesPerBlock;  // a wave per chunk
+        const int64_t all = (chunks * p.L + kWavesPerBlock - 1) / kWavesPerBlock;
+        const int64_t blocks = std::max(need, std::min(all, most));
+        hipLaunchKernelGGL((draw_kernel<false>), dim3((unsigned)blocks), dim3(kDrawBlock), lds, stream, p, 0,
+                           (int32_t)chunks, lds_alias_n);
+    }
+    return hipGetLastError();
+}
+
+template <int kGroup>
+hipError_t launch_levels_of(const LevelParams &p, bool zero_edges, int threads, size_t lds, hipStream_t stream) {
+    const void *fn = zero_edges ? (const void *)level_kernel<kGroup, true> : (const void *)level_kernel<kGroup, false>;
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const int32_t groups = (p.n + kGroup - 1) / kGroup;
+    LevelParams args = p;
+    void *kargs[] = {&args};
+    return hipLaunchKernel(fn, dim3((unsigned)((groups + 7) / 8 * 8)), dim3((unsigned)threads), kargs, lds, stream);
+}
+
+hipError_t launch_levels(const LevelParams &p, bool zero_edges, int group, int threads, int slots, hipStream_t stream) {
+    if (p.n <= 0 || p.n_levels <= 0) return hipSuccess;
+    if (threads < kLanes || threads > kLevelMaxThreads || threads % kLanes || threads % group) return hipErrorInvalidValue;
+    if (!p.dur) return hipErrorInvalidValue;
+    const size_t lds = (size_t)slots * (size_t)group * sizeof(double);
+    if (lds > kLevelLdsMaxBytes) return hipErrorInvalidValue;
+    switch (group) {
+        case 1: return launch_levels_of<1>(p, zero_edges, threads, lds, stream);
+        case 2: return launch_levels_of<2>(p, zero_edges, threads, lds, stream);
+        case 4: return launch_levels_of<4>(p, zero_edges, threads, lds, stream);
+        case 8: return launch_levels_of<8>(p, zero_edges, threads, lds, stream);
+        case 16: return launch_levels_of<16>(p, zero_edges, threads, lds, stream);
+        case 32: return launch_levels_of<32>(p, zero_edges, threads, lds, stream);
+        case 64: return launch_levels_of<64>(p, zero_edges, threads, lds, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 __global__ void reset_counter_kernel(int32_t *counter) { *counter = 0; }
 
 __global__ void philox_debug_kernel(int variant, int64_t n, const uint32_t *__restrict__ ctr,

@@ -94,6 +94,63 @@ constexpr int kWideBatch = 4;
 hipError_t launch_walk_wide(const WalkParams &p, bool injected, int32_t e0, int32_t n_events, int32_t groups,
                             hipStream_t stream);
 hipError_t launch_walk_wide_orphans(const WalkParams &p, int32_t groups, hipStream_t stream);
+// The two-pass route of short runs: every duration first (draw_kernel), then
+// the max-plus propagation level by level with the durations read back
+// (level_kernel).  Events in level order ("items"), structure of arrays, so
+// that consecutive lanes read consecutive items.
+constexpr int kLevelPreds = 4;           // predecessors an item carries inline; the rest are in `extra`
+constexpr int kLevelMaxThreads = 1024;
+constexpr int kLevelMaxGroup = 64;       // samples per workgroup: a power of two up to this
+constexpr size_t kLevelLdsMaxBytes = 160 * 1024;
+// An event and its first kLevelPreds predecessors, as four 16-byte quads
+// (LevelParams::quad): {earliest, upper}, {event, slot | count << 16, the
+// predecessors' slots, two in a word}, {edges}, {sources}.  Slots are LDS
+// slots of 15 bits (the event's own -1 if no later level reads it): a stale
+// predecessor's holds its earliest time, and positions past the last
+// predecessor name a slot that holds NaN, which never wins, and repeat the
+// first one's edge (or row 0).  An edge is a durations row, or -1: duration 0.0.  Counts
+// above kLevelPreds: the others are extra[extra_of[event]...].
+constexpr int kLevelQuads = 4;
+struct alignas(16) LevelQuad {
+    int32_t v[4];
+};
+struct LevelPred {
+    int32_t slot, edge, src;
+};
+struct LevelInit {  // a slot that holds the same value for every sample
+    double value;
+    int32_t slot, pad;
+};
+struct LevelParams {
+    const int32_t *off;      // [n_levels + 2]: items of each level, E at the end twice
+    const LevelQuad *quad;   // [kLevelQuads][E] in level order
+    const LevelPred *extra;
+    const int32_t *extra_of; // [E] by event
+    const LevelInit *init;   // [n_init]: the NaN slot, then the stale sources'
+    int32_t n_init;
+    int32_t E;
+    int32_t n_levels;
+    const double *dur;       // [L][ld], L > 0
+    int32_t n, ld;
+    double *realized;        // [E][ld]
+    int32_t *cause;          // [E][ld] or null
+    uint8_t *cause_pos;      // [E][ld] or null (as WalkParams::cause_pos)
+};
+struct DrawParams {
+    const Record *recs;  // [L]: one per link, costliest laws first
+    const DistParams *dists;
+    const AliasRec *alias;
+    int32_t n_alias;
+    int32_t L;
+    const int32_t *seeds;  // [n]
+    int32_t n, ld;
+    double *durations;     // [L][ld]
+};
+hipError_t launch_draws(const DrawParams &p, int cus, hipStream_t stream);
+// group: samples per workgroup; threads: a multiple of 64 and of group;
+// slots: LDS slots of 8 * group bytes.
+// zero_edges: some predecessor's edge is -1.
+hipError_t launch_levels(const LevelParams &p, bool zero_edges, int group, int threads, int slots, hipStream_t stream);
 hipError_t launch_copy(double *dst, const double *src, int64_t n, hipStream_t stream);
 hipError_t launch_math_debug(int fn, int64_t n, const double *x, double *out, hipStream_t stream);
 hipError_t launch_philox_debug(int variant, int64_t n, const uint32_t *ctr, const uint32_t *key, uint32_t *out,

@@ -296,7 +296,7 @@ int mcdp::event_stats_positions(mcdp_propagator &P, const double *realized, cons
         HIP_TRY(launch_event_mean(realized, (int32_t)n, (int32_t)ld, P.E, mean, s), "mean kernel");
     if (counts) {
         DeviceCopy *d = nullptr;
-        rc = ensure_device(P, d);
+        rc = device_entry(P, d);
         if (rc) return rc;
         rc = ensure_topo(P, *d);
         if (rc) return rc;
@@ -349,7 +349,7 @@ int mcdp_event_stats_device(mcdp_propagator *prop, const double *realized_dev, c
         HIP_TRY(launch_event_mean(realized_dev, (int32_t)n, (int32_t)ld, E, mean_dev, s), "mean kernel");
     if (cause_counts_dev) {
         DeviceCopy *d = nullptr;
-        rc = ensure_device(*prop, d);
+        rc = device_entry(*prop, d);
         if (rc) return rc;
         rc = ensure_topo(*prop, *d);
         if (rc) return rc;
@@ -378,11 +378,20 @@ int mcdp_run_stats_host(mcdp_propagator *prop, const int32_t *seeds, int64_t n, 
     const size_t o_mean = o_cause + 256 * (((size_t)(E * n) * cb + 255) / 256);
     const size_t o_q = o_mean + (size_t)E * 8;
     const size_t o_cnt = o_q + (size_t)E * (size_t)std::max(n_q, 0) * 8;
-    const size_t bytes = o_cnt + (size_t)(E + P) * 8;
+    size_t bytes = o_cnt + (size_t)(E + P) * 8;
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
         return fail(MCDP_E_DEVICE, "no HIP device available: statistics run on the GPU only");
     std::lock_guard<std::mutex> host_lock(prop->host_mu);
+    // a short run draws its durations first, into the workspace
+    bool two_pass = false;
+    rc = short_run(*prop, false, n, two_pass);
+    if (rc) return rc;
+    const size_t o_dur = 256 * ((bytes + 255) / 256);
+    // (within what a propagator keeps, so that no call needs memory it can
+    // only have for the faster route)
+    two_pass = two_pass && o_dur + (size_t)prop->L * (size_t)n * 8 <= kHostWorkKeepBytes;
+    if (two_pass) bytes = o_dur + (size_t)prop->L * (size_t)n * 8;
     void *buf = nullptr;
     hipStream_t st = nullptr;
     rc = host_workspace(*prop, bytes, buf, st);
@@ -395,17 +404,18 @@ int mcdp_run_stats_host(mcdp_propagator *prop, const int32_t *seeds, int64_t n, 
     auto *d_mean = reinterpret_cast<double *>(b + o_mean);
     auto *d_q = reinterpret_cast<double *>(b + o_q);
     auto *d_cnt = reinterpret_cast<int64_t *>(b + o_cnt);
+    auto *d_dur = two_pass ? reinterpret_cast<double *>(b + o_dur) : nullptr;
     e = hipMemcpyAsync(d_seeds, seeds, (size_t)n * 4, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy");
     auto *d_pos = reinterpret_cast<uint8_t *>(d_cause);
     if (!rc && pos && cause_counts) {
-        rc = run_many_positions(*prop, d_seeds, n, n, d_real, d_pos, st);
+        rc = run_many_positions(*prop, d_seeds, n, n, d_real, d_pos, st, d_dur);
         if (!rc)
             rc = event_stats_positions(*prop, d_real, d_pos, n, n, n_q, q, mean ? d_mean : nullptr,
                                        quantiles ? d_q : nullptr, d_cnt, st);
     } else {
         if (!rc)
-            rc = mcdp_run_many_device(prop, d_seeds, n, n, d_real, nullptr, cause_counts ? d_cause : nullptr, st);
+            rc = mcdp_run_many_device(prop, d_seeds, n, n, d_real, d_dur, cause_counts ? d_cause : nullptr, st);
         if (!rc)
             rc = mcdp_event_stats_device(prop, d_real, d_cause, n, n, n_q, q, mean ? d_mean : nullptr,
                                          quantiles ? d_q : nullptr, cause_counts ? d_cnt : nullptr, st);
