@@ -1,10 +1,13 @@
-"""Writes mcdp_log_table.hpp: the breakpoint table of the samplers' logarithm (log_tab in mcdp_math.hpp).
+"""Writes mcdp_log_table.hpp: the table of the samplers' logarithm (log_tab in mcdp_math.hpp).
 
-Breakpoints F_j = 1/2 + j/256, j = 0..128.  For each: 1/F_j rounded to double, and log F_j split as
-hi + lo, hi the multiple of 2^-32 nearest log F_j (so k ln2_hi + hi is exact for every binary exponent k),
-lo = log F_j - hi rounded to double.  log F_0 = -ln 2 takes the kernel's own split of ln 2 (ln2_hi, ln2_lo),
-so that log 1 = 1 * ln 2 + log(1/2) cancels to exactly 0.  Values come from the host's 80-bit long double
-logarithm (64-bit significand); hi + lo is within 2^-64 of log F_j.
+With hx the high word of x, kLogBase - hx = 2^20 m + 2^12 j + (low bits) names a scale and an interval:
+z = x 2^m lies in interval j of 256, whose middle c_j is the double of high word
+kLogBase + 1 - 2^11 - 2^12 j and low word 0 (c from 1.375 down to 0.69; 1.0 is one of them).  For each
+interval: inv_j = 1/c_j rounded to a multiple of 2^-10 (so that z inv_j - 1 needs hardly more than a double's
+53 bits and its rounding all but vanishes), and -log(inv_j) split as hi + lo, hi the multiple of 2^-32
+nearest it (so hi - m ln2_hi is exact for every binary exponent), lo the rest rounded to double.  Values
+come from the host's 80-bit long double logarithm (64-bit significand); hi + lo is within 2^-64 of
+-log(inv_j).
 
 Run: python mc_dagprop_amd/csrc/gen_log_table.py  (rewrites the header next to this file).
 """
@@ -15,9 +18,8 @@ import pathlib
 
 import numpy as np
 
-N = 129
-LN2_HI = float.fromhex("0x1.62e42feep-1")  # 0x3fe62e42fee00000, a multiple of 2^-32
-LN2_LO = 1.90821492927058770002e-10
+N = 256
+BASE = 0x3FF00000 + 0x60000 + 0x800 - 1  # the largest high word of z: 1.375 + half an interval
 
 
 def table() -> tuple[list[float], list[float], list[float]]:
@@ -25,18 +27,16 @@ def table() -> tuple[list[float], list[float], list[float]]:
     assert np.finfo(LD).nmant >= 63, "needs x87 long double"
     inv, hi, lo = [], [], []
     for j in range(N):
-        f = LD(0.5) + LD(j) / LD(256)
-        inv.append(float(1.0 / float(f)))
-        lf = np.log(f)
-        if j == 0:
-            h, l = -LN2_HI, -LN2_LO
-        else:
-            h = float(np.rint(lf * LD(2.0**32)) / LD(2.0**32))
-            l = float(lf - LD(h))
+        word = BASE + 1 - 0x800 - 0x1000 * j
+        c = float(np.array([word << 32], dtype=np.uint64).view(np.float64)[0])
+        v = float(np.rint(1024.0 / c)) / 1024.0
+        lf = -np.log(LD(v))
+        h = float(np.rint(lf * LD(2.0**32)) / LD(2.0**32))
         assert h == np.ldexp(np.rint(np.ldexp(h, 32)), -32)
+        inv.append(v)
         hi.append(h)
-        lo.append(l)
-    assert hi[-1] == 0.0 and lo[-1] == 0.0 and inv[-1] == 1.0 and inv[0] == 2.0
+        lo.append(float(lf - LD(h)))
+    assert any(v == 1.0 and h == 0.0 and l == 0.0 for v, h, l in zip(inv, hi, lo))
     return inv, hi, lo
 
 
@@ -50,12 +50,11 @@ def render() -> str:
 
     hilo = [v for pair in zip(hi, lo) for v in pair]
     return (
-        "// Generated by gen_log_table.py: breakpoints F_j = 1/2 + j/256 of log_tab (mcdp_math.hpp).\n"
-        "// kLogInvF[j] = 1/F_j rounded; log F_j = kLogHiLo[2j] + kLogHiLo[2j + 1], the first a multiple\n"
-        "// of 2^-32.\n"
+        "// Generated by gen_log_table.py: the intervals of log_tab (mcdp_math.hpp).  kLogInv[j] = 1/c_j rounded to\n"
+        "// 2^-10; -log(kLogInv[j]) = kLogHiLo[2j] + kLogHiLo[2j + 1], the first a multiple of 2^-32.\n"
         "#pragma once\n#include <hip/hip_runtime.h>\n\nnamespace mcdp {\n\n"
-        f"constexpr int kLogTableSize = {N};\n\n"
-        + arr("kLogInvF", inv, "kLogTableSize", 4) + "\n" + arr("kLogHiLo", hilo, "2 * kLogTableSize", 4)
+        f"constexpr int kLogTableSize = {N};\nconstexpr uint32_t kLogBase = 0x{BASE:08x}u;\n\n"
+        + arr("kLogInv", inv, "kLogTableSize", 4) + "\n" + arr("kLogHiLo", hilo, "2 * kLogTableSize", 4)
         + "\n}  // namespace mcdp\n"
     )
 

@@ -499,8 +499,11 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
 // LDS slots of the two-pass route: an event that a later level reads has one
 // from its own level to the last that reads it.  level_kernel writes a level's
 // results while other waves may still read for that level, so a slot is given
-// out again from the level after its last read.
+// out again from the level after its last read.  Done once, when a run first
+// asks for its route.
 void build_level_slots(mcdp_propagator &P) {
+    if (P.level_ready) return;
+    P.level_ready = true;
     const int32_t n_levels = (int32_t)P.levels.size();
     std::vector<int32_t> level((size_t)P.E, 0), last_use((size_t)P.E, -1);
     P.level_width = 0;
@@ -694,7 +697,6 @@ int compile_propagator(mcdp_propagator &P, int32_t n_events, const double *earli
     P.E = E;
     P.L = L;
     P.earliest.assign(earliest, earliest + E);
-    build_level_slots(P);
 
     // (6) default schedule.
     int32_t W, K;
@@ -918,11 +920,12 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
     d.base.slots = P.slots;
     return MCDP_OK;
 }
-// The fast kernel variant needs every read predecessor in LDS (or stale) and
-// the alias tables small enough to stage in LDS.
+// The fast kernel variant needs every read predecessor in LDS (or stale), the
+// alias tables small enough to stage in LDS, and no cap of -0 (which only a
+// max_delay of -0 gives: its cap is a v_min_f64, where -0 is below +0).
 WalkVariant walk_variant(const mcdp_propagator &P, bool injected) {
     const bool alias_fits = P.alias.size() * sizeof(AliasRec) <= kAliasLdsMaxBytes;
-    const bool fast = P.n_global == 0 && (injected || alias_fits);
+    const bool fast = P.n_global == 0 && (injected || alias_fits) && !std::signbit(P.max_delay);
     return WalkVariant{injected, fast ? kPathsFast : kPathsGeneral, P.k, P.spl};
 }
 
@@ -1019,18 +1022,22 @@ int level_group(const mcdp_propagator &P, int64_t n, int cus) {
 // Whether a run of n samples takes the two-pass route (draw_kernel, then
 // level_kernel) instead of a partial round of the walk: when its estimated time
 // is below a tile's.  The walk's tile costs the same however few of its lanes
-// and of the device's CUs are in use: 12 ns per unit of walk_cost (200 x 100
-// events, any n up to a round: 3.3 ms; 20 x 10: 93 us).  The two passes move
+// and of the device's CUs are in use: about 11.5 ns per unit of walk_cost (200 x
+// 100 events, any n up to a round: 3.0 ms; 20 x 10: 88 us), about 15 where
+// predecessors spill to global memory (60 x 250: 4.6 ms); the estimate takes a
+// tenth off, so that a run near the line walks.  The two passes move
 // the durations twice, at about 3.9 TB/s where they are bound by that, but at
 // least a level's latency per level (200 x 100, sampled: 1 sample 0.11 ms, 4,001
 // 1.20, 8,192 2.25 against 2.3 with wide steps, 12,345 3.9 against 3.3; 60 x 250:
 // 12,345 3.3 against 4.8).
-constexpr double kTileSecondsPerCost = 12e-9;
+constexpr double kTileSecondsPerCost = 10.5e-9;
+constexpr double kTileSecondsPerCostSpilled = 14e-9;
 constexpr double kLevelSeconds = 0.45e-6;       // one level of one workgroup
 constexpr double kLevelFixedSeconds = 10e-6;    // the second launch, the tables
 constexpr double kLevelBytesPerSecond = 3.9e12;
-bool level_route(const mcdp_propagator &P, bool injected, int64_t n, int cus) {
+bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus) {
     if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
+    build_level_slots(P);
     const int group = level_group(P, n, cus);
     if (group == 0) return false;
     const double per_pass = (double)group * cus;  // samples of one workgroup per CU
@@ -1039,7 +1046,8 @@ bool level_route(const mcdp_propagator &P, bool injected, int64_t n, int cus) {
     const double moved = (n > per_pass ? padded : (double)n) * (8.0 * P.L + 12.0 * P.E) / kLevelBytesPerSecond;
     const double waves = (n > per_pass ? padded / per_pass : 1.0);
     const double levels = std::max(moved, waves * kLevelSeconds * (double)P.levels.size());
-    return kLevelFixedSeconds + draws + levels < kTileSecondsPerCost * (double)P.walk_cost;
+    const double per_cost = P.n_global > 0 ? kTileSecondsPerCostSpilled : kTileSecondsPerCost;
+    return kLevelFixedSeconds + draws + levels < per_cost * (double)P.walk_cost;
 }
 
 int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injected, const int32_t *seeds,

@@ -153,8 +153,10 @@ struct mcdp_propagator {
     int64_t n_global = 0;
     bool shape_fixed = false;  // set by configure / autotune / the first launch
     bool shape_by_caller = false;  // configure chose the walk's shape: short runs keep to the walk too
-    // the two-pass route of short runs (schedule-independent): LDS slot of
-    // each event (-1: no later level reads it), slots in all, widest level
+    // the two-pass route of short runs (schedule-independent, made when first
+    // asked for): LDS slot of each event (-1: no later level reads it), slots
+    // in all, widest level
+    bool level_ready = false;
     std::vector<int32_t> level_slot;
     std::vector<std::pair<int32_t, int32_t>> level_stale;  // (source, its slot), sources ascending
     int32_t level_slots = 0, level_width = 0;

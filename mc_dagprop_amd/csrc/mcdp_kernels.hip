@@ -20,7 +20,16 @@
 // The arithmetic of propagation is FP64 add and compare-select only, in the
 // reference's order: t = realized[src] + dur; t = (upper < t) ? upper : t;
 // if (t >= best) {best = t; cause = src}; realized = (upper < best) ? upper : best.
-// std::min is (b < a) ? b : a, so a NaN candidate is never taken; no v_min_f64.
+// std::min is (b < a) ? b : a, so a NaN candidate is never taken (the fast
+// paths take v_min_f64 of a candidate that has won already, see capped_at).
+//
+// Bound by instruction issue: a wave-activity of the network workload takes
+// about 125 VALU instructions (4.3 cycles each on a SIMD, 2.4 for one- and
+// two-operand 32-bit ones) for its two samples.  200 x 100 events, 100,000
+// samples: 11.9 ms -> 11.2 with the integer-indexed logarithm, a lane's two
+// draws side by side, output rows addressed by scalar base and lane offset and
+// the cap as one instruction (63.8 GB of outputs, 5.7 TB/s; a plain fill of that
+// size runs at 6.9); 32,768 samples 3.90 -> 3.57.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -61,17 +70,53 @@ __device__ __forceinline__ uint64_t row_offset(int32_t row, uint32_t ld) { retur
 // first at equal priority, so with equal work its youngest wave would finish
 // every step last while the others wait at the step's barrier.  A wave later
 // on its SIMD (waves go to the four SIMDs in turn: rank wave / 4) counts
-// itself a further 1/16 of the step behind per rank.
-__device__ __forceinline__ void step_priority(int left, int total, int wave) {
-    const int l = left + (((wave >> 2) * total) >> 4);
-    if (4 * l > 3 * total)
+// itself a further 1/16 of the step behind per rank.  One comparison per event,
+// against the record where the next quarter begins.
+struct StepPriority {
+    int bound, quarter, prio;
+    __device__ __forceinline__ void begin(int r0, int r1, int wave) {
+        const int total = r1 - r0;
+        quarter = (total + 3) >> 2;
+        bound = r0 + quarter + (((wave >> 2) * total) >> 4);
+        prio = 3;
         __builtin_amdgcn_s_setprio(3);
-    else if (2 * l > total)
-        __builtin_amdgcn_s_setprio(2);
-    else if (4 * l > total)
-        __builtin_amdgcn_s_setprio(1);
-    else
-        __builtin_amdgcn_s_setprio(0);
+    }
+    __device__ __forceinline__ void event(int r) {
+        if (r < bound) return;
+        bound += quarter;
+        --prio;
+        if (prio == 2)
+            __builtin_amdgcn_s_setprio(2);
+        else if (prio == 1)
+            __builtin_amdgcn_s_setprio(1);
+        else
+            __builtin_amdgcn_s_setprio(0);
+    }
+};
+
+// A lane's element of an output row: the row's uniform base and the lane's
+// 32-bit byte offset, which a store takes as they are.
+template <typename T>
+__device__ __forceinline__ T *lane_ptr(T *row, uint32_t &byte) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // redefined at each use, so that it is extended there: hoisted out of the
+    // loop, the 64-bit offset would be added by an instruction of its own
+    asm volatile("" : "+v"(byte));
+#endif
+    return (T *)((char *)row + byte);
+}
+
+// min(a, b) of a candidate b that is not NaN or loses anyway: v_min_f64 keeps
+// -0 below +0, so it is (a < b) ? a : b except for a = -0 and b = +0, which the
+// host keeps away from this path.
+__device__ __forceinline__ double capped_at(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return a < b ? a : b;
+#endif
 }
 
 // Alias tables staged in LDS after the slots (fast sampled variant), so an
@@ -129,14 +174,21 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
     // Lanes past the last sample (last tile only) take over sample n - 1:
     // same seed or injected row, so they compute its values bit for bit and
     // their stores rewrite its bytes unchanged.  No store needs a lane mask.
-    uint32_t s[kSpl];
+    uint32_t at8[kSpl];  // byte of the lane's sample in the tile's part of a row of doubles
     uint32_t seed[kSpl];
+    const int32_t s0 = tile * (kLanes * kSpl);
 #pragma unroll
     for (int i = 0; i < kSpl; ++i) {
-        const int32_t si = tile * (kLanes * kSpl) + i * kLanes + lane;
-        s[i] = si < p.n ? si : p.n - 1;
-        seed[i] = kInjected ? 0u : (uint32_t)p.seeds[s[i]];
+        const int32_t si = s0 + i * kLanes + lane;
+        const int32_t s = si < p.n ? si : p.n - 1;
+        at8[i] = (uint32_t)(s - s0) * 8u;
+        seed[i] = kInjected ? 0u : (uint32_t)p.seeds[s];
     }
+    // the tile's columns of every array
+    const double *const dur_in = p.dur_in + s0;
+    double *const realized = p.realized + s0, *const durations = p.durations + s0;
+    int32_t *const cause = p.cause + s0;
+    uint8_t *const cause_pos = p.cause_pos + s0;
 
     for (int t = 0; t < p.n_steps; ++t) {
         const int r0 = step_off[t * W + wave];
@@ -147,7 +199,10 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
             // One stream of records: an event header, then its predecessors
             // in input order.  The stream ends in a padding record, so the
             // one-ahead prefetch never leaves the array.
-            Record cur = recs[r0];
+            auto rec = recs + r0;
+            Record cur = *rec;
+            StepPriority priority;
+            priority.begin(r0, r1, wave);
             double best[kSpl], upper = 0.0;
             int32_t who[kSpl], event = 0;
             int hdr = r0;  // kPos: the current event's header record (entry k is record hdr + 1 + k)
@@ -157,9 +212,9 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                 who[i] = -1;
             }
             for (int r = r0; r < r1; ++r) {
-                const Record nxt = recs[r + 1];
+                const Record nxt = *++rec;
                 if (cur.info & kInfoHeader) {
-                    step_priority(r1 - r, r1 - r0, wave);
+                    priority.event(r);
                     upper = cur.b;
                     // one vector copy per event: the caps and the final clamp
                     // select against it without rebuilding it from SGPRs
@@ -180,7 +235,7 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                             const uint64_t row = row_offset(cur.i2, ld);
 #pragma unroll
                             for (int i = 0; i < kSpl; ++i)
-                                dur[i] = __builtin_nontemporal_load(p.dur_in + row + s[i]);
+                                dur[i] = __builtin_nontemporal_load(lane_ptr(dur_in + row, at8[i]));
                         }
                     } else {
                         // an edge outside the link table is kind kNone with
@@ -190,7 +245,7 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                             const uint64_t row = row_offset(cur.i2, ld);
 #pragma unroll
                             for (int i = 0; i < kSpl; ++i)
-                                __builtin_nontemporal_store(dur[i], p.durations + row + s[i]);
+                                __builtin_nontemporal_store(dur[i], lane_ptr(durations + row, at8[i]));
                         }
                     }
                     double rs[kSpl];
@@ -199,7 +254,7 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                     } else if (kPaths == kPathsGeneral && cur.i1 == kSrcGlobal) {
                         const uint64_t row = row_offset(cur.i0, ld);
 #pragma unroll
-                        for (int i = 0; i < kSpl; ++i) rs[i] = p.realized[row + s[i]];
+                        for (int i = 0; i < kSpl; ++i) rs[i] = *lane_ptr(realized + row, at8[i]);
                     } else {
                         const double e = earliest[cur.i0];
 #pragma unroll
@@ -209,11 +264,21 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                     const int32_t tag = kPos ? r - hdr - 1 : cur.i0;
 #pragma unroll
                     for (int i = 0; i < kSpl; ++i) {
-                        double tt = rs[i] + dur[i];
-                        tt = (upper < tt) ? upper : tt;
-                        if (tt >= best[i]) {
-                            best[i] = tt;
-                            who[i] = tag;
+                        const double tt = rs[i] + dur[i];
+                        if (kPaths == kPathsFast) {
+                            // best <= upper from the start (max_delay >= 0), so
+                            // the capped candidate wins where the bare one does;
+                            // a NaN wins neither way
+                            const bool wins = tt >= best[i];
+                            const double capped = capped_at(upper, tt);
+                            best[i] = wins ? capped : best[i];
+                            who[i] = wins ? tag : who[i];
+                        } else {
+                            const double capped = (upper < tt) ? upper : tt;
+                            if (capped >= best[i]) {
+                                best[i] = capped;
+                                who[i] = tag;
+                            }
                         }
                     }
                 }
@@ -221,12 +286,14 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                     const uint64_t row = row_offset(event, ld);
 #pragma unroll
                     for (int i = 0; i < kSpl; ++i) {
-                        const double rr = (upper < best[i]) ? upper : best[i];
-                        __builtin_nontemporal_store(rr, p.realized + row + s[i]);
+                        const double rr = kPaths != kPathsFast && upper < best[i] ? upper : best[i];
+                        __builtin_nontemporal_store(rr, lane_ptr(realized + row, at8[i]));
                         if (kPos) {
-                            if (p.cause_pos) __builtin_nontemporal_store((uint8_t)who[i], p.cause_pos + row + s[i]);
+                            uint32_t at = at8[i] >> 3;
+                            if (p.cause_pos) __builtin_nontemporal_store((uint8_t)who[i], lane_ptr(cause_pos + row, at));
                         } else if (p.cause) {
-                            __builtin_nontemporal_store(who[i], p.cause + row + s[i]);
+                            uint32_t at = at8[i] >> 1;
+                            __builtin_nontemporal_store(who[i], lane_ptr(cause + row, at));
                         }
                         res[j][i] = rr;
                     }
@@ -257,8 +324,7 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
             draw(rec, seed, dur);
             const uint64_t row = row_offset(rec.i2, ld);
 #pragma unroll
-            for (int i = 0; i < kSpl; ++i)
-                __builtin_nontemporal_store(dur[i], p.durations + row + s[i]);
+            for (int i = 0; i < kSpl; ++i) __builtin_nontemporal_store(dur[i], lane_ptr(durations + row, at8[i]));
         }
     }
 }
@@ -408,9 +474,10 @@ __global__ void __launch_bounds__(kLanes) walk_wide_orphans_kernel(WalkParams p)
 // the stores before it too.
 constexpr int kDrawBlock = 256;
 constexpr int kDrawSpl = 4;
+constexpr int kDrawBlocksPerCu = 6;  // resident at once: four waves a block, one per SIMD (80 VGPRs)
 
 template <bool kLaneLinks>
-__global__ void __launch_bounds__(kDrawBlock) draw_kernel(DrawParams p, int32_t group, int32_t n_chunks,
+__global__ void __launch_bounds__(kDrawBlock, kDrawBlocksPerCu) draw_kernel(DrawParams p, int32_t group, int32_t n_chunks,
                                                           int32_t lds_alias_n) {
     extern __shared__ double lds[];
     __shared__ LogTableLds log_lds;
@@ -462,7 +529,7 @@ __global__ void __launch_bounds__(kDrawBlock) draw_kernel(DrawParams p, int32_t 
                 draw_durations<kDrawSpl>(r.info, r.a, r.b, (uint32_t)r.i2, seed, as_const_space(p.alias), dists, lt, dur);
             double *const row = p.durations + row_offset(r.i2, ld);
 #pragma unroll
-            for (int i = 0; i < kDrawSpl; ++i) row[s[i]] = dur[i];
+            for (int i = 0; i < kDrawSpl; ++i) __builtin_nontemporal_store(dur[i], row + s[i]);
         }
     }
 }
@@ -602,7 +669,7 @@ hipError_t launch_draws(const DrawParams &p, int cus, hipStream_t stream) {
     const int32_t lds_alias_n = alias_bytes <= kAliasLdsMaxBytes ? p.n_alias : 0;
     const size_t lds = lds_alias_n > 0 ? alias_bytes : 0;
     constexpr int kWavesPerBlock = kDrawBlock / kLanes;
-    const int64_t most = (int64_t)cus * 8;  // blocks resident at once, about
+    const int64_t most = (int64_t)cus * kDrawBlocksPerCu;
     if (p.n < kLanes) {
         int32_t group = 1;
         while (group < p.n) group *= 2;

@@ -26,16 +26,16 @@ __device__ __forceinline__ double fma_k(double p, double z, double c) {
 #endif
 }
 
-// The breakpoint table of log_tab (the lookups are per lane): kLogInvF and
-// kLogHiLo from mcdp_log_table.hpp, written by gen_log_table.py.  Kernels
-// that sample many activities per workgroup stage it in LDS; the others read
-// it where it lies (global_log_table).
+// The table of log_tab (the lookups are per lane): kLogInv and kLogHiLo from
+// mcdp_log_table.hpp, written by gen_log_table.py.  Kernels that sample many
+// activities per workgroup stage it in LDS (6 KB); the others read it where it
+// lies (global_log_table).
 struct LogTable {
-    const double *inv;    // [kLogTableSize]: 1/F_j rounded
-    const double2 *hilo;  // [kLogTableSize]: log F_j = hi + lo, hi a multiple of 2^-32
+    const double *inv;    // [kLogTableSize]: 1/c_j rounded to 2^-10
+    const double2 *hilo;  // [kLogTableSize]: -log(inv_j) = hi + lo, hi a multiple of 2^-32
 };
 __device__ __forceinline__ LogTable global_log_table() {
-    return LogTable{kLogInvF, reinterpret_cast<const double2 *>(kLogHiLo)};
+    return LogTable{kLogInv, reinterpret_cast<const double2 *>(kLogHiLo)};
 }
 struct LogTableLds {
     double inv[kLogTableSize];
@@ -46,76 +46,119 @@ struct LogTableLds {
 // table visible to all waves.
 __device__ __forceinline__ void stage_log_table(LogTableLds &t) {
     for (int i = threadIdx.x; i < kLogTableSize; i += blockDim.x) {
-        t.inv[i] = kLogInvF[i];
+        t.inv[i] = kLogInv[i];
         t.hilo[i] = double2{kLogHiLo[2 * i], kLogHiLo[2 * i + 1]};
     }
 }
 
-// Natural logarithm of a positive finite x, table-driven (P. T. P. Tang,
+// Natural logarithms of N positive normal x, table-driven (P. T. P. Tang,
 // "Table-driven implementation of the logarithm function in IEEE
-// floating-point arithmetic", ACM TOMS 16(4), 1990):
-// x = 2^k m with m in [1/2, 1); F = 1/2 + j/256 the breakpoint nearest m;
-// log x = k ln2 + log F + log(1 + r) with r = (m - F)/F, |r| <= 2^-8.
-//   * m - F is exact (Sterbenz); r = (m - F) * (1/F) carries two roundings,
-//     i.e. ~2^-60 absolute;
-//   * log(1 + r) = r + r^2 P(r), Taylor to r^7 (remainder < 2^-67);
-//   * k ln2_hi + hi is exact (both multiples of 2^-32, sum below 2^10), and
-//     the small terms k ln2_lo + lo + log(1 + r) are added to it last.
-// At x = 1 (k = 1, F = 1/2, log F = -ln2_hi - ln2_lo) both parts cancel to 0;
-// near 1 from below F = 1 and the result is log(1 + r) alone, so the
-// relative error stays within an ulp there too.
-__device__ __forceinline__ double log_tab(double x, const LogTable &t) {
-    const double m = __builtin_amdgcn_frexp_mant(x);  // [1/2, 1)
-    const int k = __builtin_amdgcn_frexp_exp(x);
-    const double jd = __builtin_rint(__builtin_fma(m, 256.0, -128.0));  // exact argument; j in [0, 128]
-    const int j = (int)jd;
-    const double F = __builtin_fma(jd, 1.0 / 256.0, 0.5);  // exact
-    const double r = (m - F) * t.inv[j];
-    const double2 lf = t.hilo[j];
-    const double r2 = r * r;
-    double p = 1.0 / 7.0;
-    p = fma_k(p, r, -1.0 / 6.0);
-    p = fma_k(p, r, 1.0 / 5.0);
-    p = fma_k(p, r, -1.0 / 4.0);
-    p = fma_k(p, r, 1.0 / 3.0);
-    p = __builtin_fma(p, r, -0.5);
-    const double log1p_r = __builtin_fma(r2, p, r);
-    const double kd = (double)k;
+// floating-point arithmetic", ACM TOMS 16(4), 1990), the scale and interval
+// taken from x's high word with integer operations (half an FP64 operation's
+// issue time each, against frexp, rint and conversions): z = x 2^m in (0.69,
+// 1.38), c the middle of z's interval of 256, inv = 1/c rounded to 2^-10;
+// log x = -m ln2 - log(inv) + log(1 + r) with r = z inv - 1, |r| <= 2^-8.7.
+//   * r is one fma, and exact but for its last bits (a multiple of 2^-63);
+//   * log(1 + r) = r + r^2 P(r), Taylor to r^6 (remainder < 2^-55 of r);
+//   * hi - m ln2_hi is exact (both multiples of 2^-32, sum below 2^10), and
+//     the small terms lo - m ln2_lo + log(1 + r) are added to it last.
+// c = 1 is the middle of an interval, so near 1 the result is log(1 + r) alone
+// and its relative error stays within an ulp; log 1 = 0.  Measured against
+// extended precision: at most 0.78 ulp for uniforms, 0.98 ulp in (1 - 2^-8, 1).
+// The N logarithms advance step by step together: a wave issues independent
+// instructions back to back, and a dependent one half as often.
+template <int N>
+__device__ __forceinline__ void log_tab_n(const double (&x)[N], const LogTable &t, double (&out)[N]) {
+    double kd[N], z[N], inv[N];
+    double2 lf[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t d = kLogBase - (uint32_t)__double2hiint(x[i]);
+        const int m = (int)d >> 20;
+        const uint32_t j = (d >> 12) & 255u;
+        inv[i] = t.inv[j];
+        lf[i] = t.hilo[j];
+        z[i] = __builtin_amdgcn_ldexp(x[i], m);
+        kd[i] = (double)m;
+    }
     constexpr double ln2_hi = 6.93147180369123816490e-01;  // 0x3fe62e42fee00000
     constexpr double ln2_lo = 1.90821492927058770002e-10;
-    const double hi = __builtin_fma(kd, ln2_hi, lf.x);
-    const double lo = __builtin_fma(kd, ln2_lo, lf.y) + log1p_r;
-    return hi + lo;
+    double r[N], p[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        r[i] = __builtin_fma(z[i], inv[i], -1.0);
+        p[i] = -1.0 / 6.0;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = fma_k(p[i], r[i], 1.0 / 5.0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = fma_k(p[i], r[i], -1.0 / 4.0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = fma_k(p[i], r[i], 1.0 / 3.0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = __builtin_fma(p[i], r[i], -0.5);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const double log1p_r = __builtin_fma(r[i] * r[i], p[i], r[i]);
+        const double hi = __builtin_fma(-kd[i], ln2_hi, lf[i].x);
+        const double lo = __builtin_fma(-kd[i], ln2_lo, lf[i].y) + log1p_r;
+        out[i] = hi + lo;
+    }
+}
+__device__ __forceinline__ double log_tab(double x, const LogTable &t) {
+    const double v[1] = {x};
+    double out[1];
+    log_tab_n<1>(v, t, out);
+    return out[0];
 }
 
-// cos(2 pi u) for u in [0, 1], to within ~3e-16 absolute.
+// cos(2 pi u) for u in [0, 1], to within ~3e-16 absolute, N at a time.
 // Reduce to w in [0, 1/4] by the symmetries of cosine (period 1, even,
 // cos(pi - a) = -cos a), then the Taylor polynomial of cos in a = 2 pi w,
 // |a| <= pi/2, to degree 22 (remainder (pi/2)^24 / 24! < 1e-22).  Near
 // a = pi/2 the result is small and its error is absolute, which is what the
 // samplers need (they use cos as a factor of a normal deviate).
-__device__ __forceinline__ double cos2pi_fast(double u) {
-    double w = u - __builtin_rint(u);  // [-1/2, 1/2]
-    w = __builtin_fabs(w);             // cos is even
-    const bool neg = w > 0.25;         // cos(2pi w) = -cos(2pi (1/2 - w))
-    w = neg ? 0.5 - w : w;             // [0, 1/4]
+template <int N>
+__device__ __forceinline__ void cos2pi_n(const double (&u)[N], double (&out)[N]) {
     constexpr double two_pi = 6.28318530717958647693;
-    const double a = w * two_pi;
-    const double a2 = a * a;
-    // cos a = sum (-1)^n a^{2n} / (2n)!
-    double c = -1.0 / 1.1240007277776077e21;            // -1/22!
-    c = fma_k(c, a2, 1.0 / 2432902008176640000.0);  //  1/20!
-    c = fma_k(c, a2, -1.0 / 6402373705728000.0);    // -1/18!
-    c = fma_k(c, a2, 1.0 / 20922789888000.0);   //  1/16!
-    c = fma_k(c, a2, -1.0 / 87178291200.0);     // -1/14!
-    c = fma_k(c, a2, 1.0 / 479001600.0);        //  1/12!
-    c = fma_k(c, a2, -1.0 / 3628800.0);         // -1/10!
-    c = fma_k(c, a2, 1.0 / 40320.0);            //  1/8!
-    c = fma_k(c, a2, -1.0 / 720.0);             // -1/6!
-    c = fma_k(c, a2, 1.0 / 24.0);               //  1/4!
-    c = __builtin_fma(c, a2, -0.5);                    // -1/2!
-    c = __builtin_fma(c, a2, 1.0);
-    return neg ? -c : c;
+    constexpr double q[10] = {1.0 / 24.0,                        //  1/4!
+                              -1.0 / 720.0,                      // -1/6!
+                              1.0 / 40320.0,                     //  1/8!
+                              -1.0 / 3628800.0,                  // -1/10!
+                              1.0 / 479001600.0,                 //  1/12!
+                              -1.0 / 87178291200.0,              // -1/14!
+                              1.0 / 20922789888000.0,            //  1/16!
+                              -1.0 / 6402373705728000.0,         // -1/18!
+                              1.0 / 2432902008176640000.0,       //  1/20!
+                              -1.0 / 1.1240007277776077e21};     // -1/22!
+    double a2[N], c[N];
+    bool neg[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        double w = u[i] - __builtin_rint(u[i]);  // [-1/2, 1/2]
+        w = __builtin_fabs(w);                   // cos is even
+        neg[i] = w > 0.25;                       // cos(2pi w) = -cos(2pi (1/2 - w))
+        w = neg[i] ? 0.5 - w : w;                // [0, 1/4]
+        const double a = w * two_pi;
+        a2[i] = a * a;
+        c[i] = q[9];
+    }
+#pragma unroll
+    for (int k = 8; k >= 0; --k)
+#pragma unroll
+        for (int i = 0; i < N; ++i) c[i] = fma_k(c[i], a2[i], q[k]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        c[i] = __builtin_fma(c[i], a2[i], -0.5);
+        c[i] = __builtin_fma(c[i], a2[i], 1.0);
+        out[i] = neg[i] ? -c[i] : c[i];
+    }
+}
+__device__ __forceinline__ double cos2pi_fast(double u) {
+    const double v[1] = {u};
+    double out[1];
+    cos2pi_n<1>(v, out);
+    return out[0];
 }
 
 // e^x for x <= 0 down to about -745 (the only range the samplers use):

@@ -60,38 +60,47 @@ struct Words2 {
     uint32_t x, y;
 };
 
-// Philox-4x32-10.  A 32x32->64 product is one v_mad_u64_u32.
-__device__ __forceinline__ Words4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
-                                                uint32_t k1) {
+// Philox-4x32-10 and -2x32-10 of N counters under one key, the N rounds side
+// by side (see log_tab_n).  A 32x32->64 product is one v_mad_u64_u32.
+template <int N>
+__device__ __forceinline__ void philox4x32_10_n(Words4 (&c)[N], uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         if (r) {
             k0 += kPhiloxW0;
             k1 += kPhiloxW1;
         }
-        const uint64_t p0 = (uint64_t)kPhiloxM4a * c0;
-        const uint64_t p1 = (uint64_t)kPhiloxM4b * c2;
-        const uint32_t y0 = xor3((uint32_t)(p1 >> 32), c1, k0);
-        const uint32_t y2 = xor3((uint32_t)(p0 >> 32), c3, k1);
-        c1 = (uint32_t)p1;
-        c3 = (uint32_t)p0;
-        c0 = y0;
-        c2 = y2;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint64_t p0 = (uint64_t)kPhiloxM4a * c[i].x;
+            const uint64_t p1 = (uint64_t)kPhiloxM4b * c[i].z;
+            c[i] = Words4{xor3((uint32_t)(p1 >> 32), c[i].y, k0), (uint32_t)p1, xor3((uint32_t)(p0 >> 32), c[i].w, k1),
+                          (uint32_t)p0};
+        }
     }
-    return Words4{c0, c1, c2, c3};
 }
-
-// Philox-2x32-10.
-__device__ __forceinline__ Words2 philox2x32_10(uint32_t c0, uint32_t c1, uint32_t k) {
+template <int N>
+__device__ __forceinline__ void philox2x32_10_n(Words2 (&c)[N], uint32_t k) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         if (r) k += kPhiloxW0;
-        const uint64_t p = (uint64_t)kPhiloxM2 * c0;
-        const uint32_t y0 = xor3((uint32_t)(p >> 32), k, c1);
-        c1 = (uint32_t)p;
-        c0 = y0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint64_t p = (uint64_t)kPhiloxM2 * c[i].x;
+            c[i] = Words2{xor3((uint32_t)(p >> 32), k, c[i].y), (uint32_t)p};
+        }
     }
-    return Words2{c0, c1};
+}
+__device__ __forceinline__ Words4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
+                                                uint32_t k1) {
+    Words4 c[1] = {{c0, c1, c2, c3}};
+    philox4x32_10_n<1>(c, k0, k1);
+    return c[0];
+}
+__device__ __forceinline__ Words2 philox2x32_10(uint32_t c0, uint32_t c1, uint32_t k) {
+    Words2 c[1] = {{c0, c1}};
+    philox2x32_10_n<1>(c, k);
+    return c[0];
 }
 
 // ---- uniforms ---------------------------------------------------------------
@@ -104,8 +113,6 @@ __device__ __forceinline__ double bits53(uint32_t hi, uint32_t lo) {
 __device__ __forceinline__ double u01_open0(uint32_t hi, uint32_t lo) {
     return __builtin_fma((double)(hi >> 11), 0x1p-21, __builtin_fma((double)lo, 0x1p-53, 0x1p-53));
 }
-// m 2^-53, in [0, 1).
-__device__ __forceinline__ double u01(uint32_t hi, uint32_t lo) { return bits53(hi, lo) * 0x1p-53; }
 // (w + 1/2) 2^-32, in (0, 1): 32-bit resolution, used for an angle and for
 // the acceptance test of Marsaglia-Tsang.
 __device__ __forceinline__ double u01_mid32(uint32_t w) { return ((double)w + 0.5) * 0x1p-32; }
@@ -123,6 +130,20 @@ __device__ __forceinline__ Words2 draw_words2(uint32_t edge, uint32_t seed, uint
 }
 __device__ __forceinline__ Words4 draw_words4(uint32_t edge, uint32_t seed, uint32_t attempt, uint32_t tag) {
     return philox4x32_10(seed, tag, attempt, 0u, edge, 0u);
+}
+
+// The same for a lane's N samples, first attempt.
+template <int N>
+__device__ __forceinline__ void draw_words2_n(uint32_t edge, const uint32_t (&seed)[N], Words2 (&w)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = Words2{seed[i], kTagMain};
+    philox2x32_10_n<N>(w, edge);
+}
+template <int N>
+__device__ __forceinline__ void draw_words4_n(uint32_t edge, const uint32_t (&seed)[N], Words4 (&w)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = Words4{seed[i], kTagMain, 0u, 0u};
+    philox4x32_10_n<N>(w, edge, 0u);
 }
 
 // ---- per-kind draws of the multiplier X (or the absolute extra) -------------
@@ -217,16 +238,21 @@ __device__ __forceinline__ void draw_durations(uint32_t info, double dmin, doubl
             const uint64_t packed = (uint64_t)__double_as_longlong(p0);  // (n, table_off)
             const int n = (int)(uint32_t)packed;
             const int table_off = (int)(uint32_t)(packed >> 32);
+            const double scale = (double)n * 0x1p-53;  // u01(m) n = m scale: one rounding either way
+            Words2 w[N];
+            draw_words2_n<N>(edge, seed, w);
+            double frac[N];
+            AliasRec rec[N];
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                const Words2 w = draw_words2(edge, seed[i], kTagMain);
-                const double xn = u01(w.x, w.y) * (double)n;
+                const double xn = bits53(w[i].x, w[i].y) * scale;
                 int b = (int)xn;
                 b = (b >= n) ? n - 1 : b;
-                const double frac = xn - (double)b;
-                const AliasRec rec = alias[table_off + b];
-                X[i] = (frac < rec.prob) ? rec.v_self : rec.v_alias;
+                frac[i] = xn - (double)b;
+                rec[i] = alias[table_off + b];
             }
+#pragma unroll
+            for (int i = 0; i < N; ++i) X[i] = (frac[i] < rec[i].prob) ? rec[i].v_self : rec[i].v_alias;
             if (kind == kEmpiricalAbs) {
 #pragma unroll
                 for (int i = 0; i < N; ++i) dur[i] = dmin + X[i];
@@ -239,40 +265,57 @@ __device__ __forceinline__ void draw_durations(uint32_t info, double dmin, doubl
 #pragma unroll
             for (int i = 0; i < N; ++i) X[i] = p0;
             break;
-        case kExpInf:  // inversion: X = -mean log U, U in (0, 1]
+        case kExpInf: {  // inversion: X = -mean log U, U in (0, 1]
+            Words2 w[N];
+            draw_words2_n<N>(edge, seed, w);
+            double u[N], l[N];
 #pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const Words2 w = draw_words2(edge, seed[i], kTagMain);
-                X[i] = -p0 * log_tab(u01_open0(w.x, w.y), lt);
-            }
+            for (int i = 0; i < N; ++i) u[i] = u01_open0(w[i].x, w[i].y);
+            log_tab_n<N>(u, lt, l);
+#pragma unroll
+            for (int i = 0; i < N; ++i) X[i] = -p0 * l[i];
             break;
+        }
         case kExpTrunc: {
             // Inversion of the CDF truncated at m: U' = q + (1 - q) U is uniform on
             // (q, 1] with q = e^{-m/mean}, and X = -mean log U' lies in [0, m].
             const DistParams D = dists[(info >> kInfoDistShift) & kInfoDistMask];
+            Words2 w[N];
+            draw_words2_n<N>(edge, seed, w);
+            double u[N], l[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) u[i] = __builtin_fma(u01_open0(w[i].x, w[i].y), D.p[3], D.p[1]);
+            log_tab_n<N>(u, lt, l);
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                const Words2 w = draw_words2(edge, seed[i], kTagMain);
-                const double u = __builtin_fma(u01_open0(w.x, w.y), D.p[3], D.p[1]);
-                const double x = -p0 * log_tab(u, lt);
+                const double x = -p0 * l[i];
                 X[i] = (x > D.p[2]) ? D.p[2] : x;
             }
             break;
         }
         default: {
             if (!(info & kInfoTruncated) && kind == kGammaErlang2) {  // sum of two unit exponentials
+                Words4 w[N];
+                draw_words4_n<N>(edge, seed, w);
+                double u[N], l[N];
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    const Words4 w = draw_words4(edge, seed[i], 0u, kTagMain);
-                    X[i] = -p0 * log_tab(u01_open0(w.x, w.y) * u01_open0(w.z, w.w), lt);
-                }
+                for (int i = 0; i < N; ++i) u[i] = u01_open0(w[i].x, w[i].y) * u01_open0(w[i].z, w[i].w);
+                log_tab_n<N>(u, lt, l);
+#pragma unroll
+                for (int i = 0; i < N; ++i) X[i] = -p0 * l[i];
             } else if (!(info & kInfoTruncated) && kind == kGammaHalf) {  // Exp(1) cos^2(2 pi U)
+                Words4 w[N];
+                draw_words4_n<N>(edge, seed, w);
+                double u[N], v[N], l[N], cs[N];
 #pragma unroll
                 for (int i = 0; i < N; ++i) {
-                    const Words4 w = draw_words4(edge, seed[i], 0u, kTagMain);
-                    const double cs = cos2pi_fast(u01_mid32(w.z));
-                    X[i] = p0 * (-log_tab(u01_open0(w.x, w.y), lt) * (cs * cs));
+                    u[i] = u01_open0(w[i].x, w[i].y);
+                    v[i] = u01_mid32(w[i].z);
                 }
+                log_tab_n<N>(u, lt, l);
+                cos2pi_n<N>(v, cs);
+#pragma unroll
+                for (int i = 0; i < N; ++i) X[i] = p0 * (-l[i] * (cs[i] * cs[i]));
             } else {
                 const DistParams D = dists[(info >> kInfoDistShift) & kInfoDistMask];
 #pragma unroll

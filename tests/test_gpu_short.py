@@ -11,7 +11,7 @@ import pytest
 import dags as D
 import oracle
 from mc_dagprop_amd import capi
-from mc_dagprop_amd.workloads import layered_vectorized, network_dists, seeded_network_dists
+from mc_dagprop_amd.workloads import FlatDag, layered_vectorized, network_dists, seeded_network_dists
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,21 @@ def test_two_pass_statistics_match_rows(gpu, n: int) -> None:
     np.testing.assert_array_equal(bits(mean), bits(m2))
     np.testing.assert_array_equal(bits(quant), bits(q2))
     np.testing.assert_array_equal(counts, c2)
+
+
+@pytest.mark.parametrize("configured", [False, True])
+def test_signed_zero_caps(gpu, configured: bool) -> None:
+    """max_delay -0 makes caps of -0, where the smaller of -0 and +0 is not what the comparison keeps."""
+    events = [(-0.0, 9.0, 0.0), (0.0, 9.0, 0.0), (-0.0, 9.0, 0.0), (-0.0, 9.0, 0.0)]
+    acts = {(0, 1): (0, 0.0, 0), (0, 2): (1, 0.0, 0), (1, 3): (2, 0.0, 0), (2, 3): (3, 0.0, 0)}
+    prec = [(1, [(0, 0)]), (2, [(0, 1)]), (3, [(1, 2), (2, 3)])]
+    dag = FlatDag.from_lists(events, acts, prec, -0.0)
+    vals = np.array([0.0, -0.0, 1.0, -1.0, np.nan])
+    dur = np.stack(np.meshgrid(vals, vals, vals, vals), -1).reshape(-1, 4)
+    P = capi.Propagator(dag)
+    if configured:
+        P.configure(4, 4, 2)
+    r, c = P.propagate(dur)
+    ro, co = oracle.OracleCtx(dag).propagate(dur)
+    np.testing.assert_array_equal(bits(r), bits(ro))
+    np.testing.assert_array_equal(c, co)
