@@ -166,7 +166,7 @@ int prepare(mcdp_batch *b, const int32_t *const *seeds_dev, const int64_t *n, co
             (void)hipFree(b->dev);
             b->dev = nullptr;
         }
-        hipError_t e = hipMalloc(&b->dev, bytes);
+        hipError_t e = device_malloc(&b->dev, bytes);
         if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (batch): ") + hipGetErrorString(e));
         b->dev_bytes = bytes;
         b->device = device;
@@ -306,7 +306,7 @@ int mcdp_batch_stats_host(mcdp_batch *b, const int32_t *const *seeds, const int6
             b->stats_work = nullptr;
             b->stats_bytes = 0;
         }
-        hipError_t e = hipMalloc(&b->stats_work, need);
+        hipError_t e = device_malloc(&b->stats_work, need);
         if (e != hipSuccess) {
             b->stats_work = nullptr;
             return fail(MCDP_E_NOMEM, std::string("hipMalloc (batch statistics): ") + hipGetErrorString(e));

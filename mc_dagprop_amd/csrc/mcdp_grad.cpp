@@ -312,7 +312,7 @@ int ensure_reverse(mcdp_propagator &P, DeviceCopy &d) {
     put(o_moff, R.map_off.data(), R.map_off.size() * 4);
     put(o_mcol, R.map_col.data(), R.map_col.size() * 4);
     void *blob = nullptr;
-    hipError_t e = hipMalloc(&blob, total);
+    hipError_t e = device_malloc(&blob, total);
     if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (reverse plan): ") + hipGetErrorString(e));
     e = hipMemcpy(blob, host.data(), total, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -353,7 +353,7 @@ int ensure_workspace(DeviceCopy &d, size_t bytes) {
         d.rev_work = nullptr;
         d.rev_work_bytes = 0;
     }
-    hipError_t e = hipMalloc(&d.rev_work, bytes);
+    hipError_t e = device_malloc(&d.rev_work, bytes);
     if (e != hipSuccess) {
         d.rev_work = nullptr;
         return fail(MCDP_E_NOMEM, std::string("hipMalloc (gradient workspace): ") + hipGetErrorString(e));

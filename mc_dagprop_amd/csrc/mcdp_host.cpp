@@ -792,7 +792,7 @@ class Upload {
     }
     int send(void *&blob) {
         blob = nullptr;
-        hipError_t e = hipMalloc(&blob, std::max<size_t>(host_.size(), 256));
+        hipError_t e = device_malloc(&blob, std::max<size_t>(host_.size(), 256));
         if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
         e = hipMemcpy(blob, host_.data(), host_.size(), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
@@ -881,7 +881,7 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
     put(o_earl, P.earliest.data(), P.earliest.size() * sizeof(double));
     put(o_evrec, P.ev_rec.data(), P.ev_rec.size() * sizeof(int32_t));
     void *blob = nullptr;
-    hipError_t e = hipMalloc(&blob, total);
+    hipError_t e = device_malloc(&blob, total);
     if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
     e = hipMemcpy(blob, host.data(), total, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -1226,6 +1226,108 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
 
 }  // namespace
 
+namespace {
+
+// Workspaces of more than kHostWorkKeepBytes between calls.  Giving such memory
+// back and having it again costs 27 ms per GB (the driver clears it): 171 ms a
+// call for the statistics of 32,768 samples of the network DAG, whose kernels
+// take 5.  So the process keeps some: per device at most an eighth of its
+// memory in all, and only while a quarter of it stays free; the oldest goes
+// first.  A propagator's calls and the next propagator's share them (a call
+// owns its workspace from taking it to giving it back, its stream idle), they
+// are freed with the propagator that used them last, and before any allocation
+// of this library fails.
+struct LargePool {
+    struct Entry {
+        int device;
+        void *buf;
+        size_t bytes;
+        const void *owner;
+    };
+    std::mutex mu;
+    std::vector<Entry> kept;  // oldest first
+
+    static void release(const Entry &e) {
+        int cur = -1;
+        (void)hipGetDevice(&cur);
+        (void)hipSetDevice(e.device);
+        (void)hipFree(e.buf);
+        if (cur >= 0) (void)hipSetDevice(cur);
+    }
+    // The smallest kept workspace of at least `need` bytes, or null.
+    void *take(int device, size_t need, size_t &bytes) {
+        std::lock_guard<std::mutex> lock(mu);
+        size_t best = kept.size();
+        for (size_t i = 0; i < kept.size(); ++i)
+            if (kept[i].device == device && kept[i].bytes >= need && (best == kept.size() || kept[i].bytes < kept[best].bytes))
+                best = i;
+        if (best == kept.size()) return nullptr;
+        void *buf = kept[best].buf;
+        bytes = kept[best].bytes;
+        kept.erase(kept.begin() + (std::ptrdiff_t)best);
+        return buf;
+    }
+    // Keeps or frees an idle workspace of the current device.
+    void give(int device, void *buf, size_t bytes, const void *owner) {
+        std::lock_guard<std::mutex> lock(mu);
+        const Entry e{device, buf, bytes, owner};
+        size_t free_bytes = 0, total = 0;
+        if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > total / 8 || free_bytes < total / 4) {
+            release(e);
+            return;
+        }
+        size_t sum = bytes;
+        for (const Entry &k : kept) sum += k.device == device ? k.bytes : 0;
+        for (size_t i = 0; i < kept.size() && sum > total / 8;) {
+            if (kept[i].device != device) {
+                ++i;
+                continue;
+            }
+            sum -= kept[i].bytes;
+            release(kept[i]);
+            kept.erase(kept.begin() + (std::ptrdiff_t)i);
+        }
+        kept.push_back(e);
+    }
+    // Frees every kept workspace that `which` names; whether there was one.
+    template <typename F>
+    bool drop(F &&which) {
+        std::lock_guard<std::mutex> lock(mu);
+        bool any = false;
+        for (size_t i = 0; i < kept.size();) {
+            if (!which(kept[i])) {
+                ++i;
+                continue;
+            }
+            release(kept[i]);
+            kept.erase(kept.begin() + (std::ptrdiff_t)i);
+            any = true;
+        }
+        return any;
+    }
+};
+// (never destroyed: propagators may outlive static objects)
+LargePool &large_pool() {
+    static LargePool *const pool = new LargePool;
+    return *pool;
+}
+
+}  // namespace
+
+hipError_t mcdp::device_malloc(void **ptr, size_t bytes) {
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipSuccess) return e;
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return e;
+    if (!large_pool().drop([&](const LargePool::Entry &k) { return k.device == device; })) return e;
+    (void)hipGetLastError();
+    return hipMalloc(ptr, bytes);
+}
+
+void mcdp::large_pool_drop(const void *owner) {
+    (void)large_pool().drop([&](const LargePool::Entry &k) { return k.owner == owner; });
+}
+
 int mcdp::host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_t &stream) {
     int device = 0;
     HIP_TRY(hipGetDevice(&device), "hipGetDevice");
@@ -1239,6 +1341,20 @@ int mcdp::host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_
         P.host_work.push_back(h);
         hw = &P.host_work.back();
     }
+    stream = hw->stream;
+    if (need > kHostWorkKeepBytes) {
+        hw->large = large_pool().take(device, need, hw->large_bytes);
+        if (!hw->large) {
+            hipError_t e = device_malloc(&hw->large, need);
+            if (e != hipSuccess) {
+                hw->large = nullptr;
+                return fail(MCDP_E_NOMEM, std::string("hipMalloc (host-call workspace): ") + hipGetErrorString(e));
+            }
+            hw->large_bytes = need;
+        }
+        buf = hw->large;
+        return MCDP_OK;
+    }
     if (hw->bytes < need) {
         if (hw->buf) {
             (void)hipStreamSynchronize(hw->stream);  // idle already: every call ends by waiting on it
@@ -1247,7 +1363,7 @@ int mcdp::host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_
             hw->buf = nullptr;
             hw->bytes = 0;
         }
-        hipError_t e = hipMalloc(&hw->buf, std::max<size_t>(need, 256));
+        hipError_t e = device_malloc(&hw->buf, std::max<size_t>(need, 256));
         if (e != hipSuccess) {
             hw->buf = nullptr;
             return fail(MCDP_E_NOMEM, std::string("hipMalloc (host-call workspace): ") + hipGetErrorString(e));
@@ -1255,7 +1371,6 @@ int mcdp::host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_
         hw->bytes = std::max<size_t>(need, 256);
     }
     buf = hw->buf;
-    stream = hw->stream;
     return MCDP_OK;
 }
 
@@ -1263,12 +1378,11 @@ void mcdp::host_workspace_trim(mcdp_propagator &P) {
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return;
     for (auto &h : P.host_work)
-        if (h.device == device && h.buf && h.bytes > kHostWorkKeepBytes) {
+        if (h.device == device && h.large) {
             (void)hipStreamSynchronize(h.stream);
-            h.drop_graph();
-            (void)hipFree(h.buf);
-            h.buf = nullptr;
-            h.bytes = 0;
+            large_pool().give(device, h.large, h.large_bytes, &P);
+            h.large = nullptr;
+            h.large_bytes = 0;
         }
 }
 
@@ -2013,7 +2127,7 @@ int mcdp_propagator_autotune(mcdp_propagator *prop, int64_t n_samples, int32_t *
     for (int64_t i = 0; i < n; ++i) hseeds[(size_t)i] = (int32_t)i;
     void *buf = nullptr;
     const size_t bytes = align_up((size_t)n * 4, 256) + (size_t)n * (size_t)(12 * E + 8 * L);
-    hipError_t e = hipMalloc(&buf, bytes);
+    hipError_t e = device_malloc(&buf, bytes);
     if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (autotune): ") + hipGetErrorString(e));
     auto *b = static_cast<unsigned char *>(buf);
     int32_t *d_seeds = reinterpret_cast<int32_t *>(b);
@@ -2228,7 +2342,7 @@ int mcdp_device_count(int *count) {
 }
 int mcdp_malloc(void **ptr, size_t bytes) {
     if (!ptr) return fail(MCDP_E_INVALID, "ptr is null");
-    hipError_t e = hipMalloc(ptr, bytes);
+    hipError_t e = device_malloc(ptr, bytes);
     return e == hipSuccess ? MCDP_OK : fail(MCDP_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
 }
 int mcdp_free(void *ptr) {
@@ -2331,7 +2445,7 @@ int mcdp_debug_philox(int variant, int64_t n, const uint32_t *ctr, const uint32_
     const size_t cw = (size_t)variant, kw = (size_t)(variant / 2);
     uint32_t *d = nullptr;
     const size_t bytes = sizeof(uint32_t) * (size_t)n * (cw + kw + cw);
-    HIP_TRY(hipMalloc(&d, bytes), "hipMalloc");
+    HIP_TRY(device_malloc((void **)&d, bytes), "hipMalloc");
     uint32_t *dc = d, *dk = d + (size_t)n * cw, *dout = dk + (size_t)n * kw;
     hipError_t e = hipMemcpy(dc, ctr, sizeof(uint32_t) * n * cw, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(dk, key, sizeof(uint32_t) * n * kw, hipMemcpyHostToDevice);
@@ -2350,7 +2464,7 @@ int mcdp_debug_math(int fn, int64_t n, const double *x, double *out) {
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) return fail(MCDP_E_DEVICE, "no HIP device available");
     if (n == 0) return MCDP_OK;
     double *d = nullptr;
-    HIP_TRY(hipMalloc(&d, sizeof(double) * 2 * (size_t)n), "hipMalloc");
+    HIP_TRY(device_malloc((void **)&d, sizeof(double) * 2 * (size_t)n), "hipMalloc");
     hipError_t e = hipMemcpy(d, x, sizeof(double) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_math_debug(fn, n, d, d + n, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();

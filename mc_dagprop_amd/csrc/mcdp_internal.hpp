@@ -104,6 +104,8 @@ struct HostWork {
     int device = -1;
     void *buf = nullptr;
     size_t bytes = 0;
+    void *large = nullptr;  // one call's workspace of more than kHostWorkKeepBytes (host_workspace)
+    size_t large_bytes = 0;
     hipStream_t stream = nullptr;
     // Short runs: the launches of a key seen twice in a row are captured into
     // a graph, replayed while the key stays (one graph launch instead of a
@@ -124,6 +126,14 @@ struct PredEntry {
     bool stale;  // read before src is evaluated in the reference's order
 };
 
+}  // namespace mcdp
+
+namespace mcdp {
+// hipMalloc that gives the large workspaces kept for later calls back to the
+// device before it reports that memory is out.
+hipError_t device_malloc(void **ptr, size_t bytes);
+// Frees the large workspaces whose last user was `owner`.
+void large_pool_drop(const void *owner);
 }  // namespace mcdp
 
 struct mcdp_propagator {
@@ -207,6 +217,7 @@ struct mcdp_propagator {
             if (h.stream) (void)hipStreamDestroy(h.stream);
             if (cur >= 0) (void)hipSetDevice(cur);
         }
+        mcdp::large_pool_drop(this);
     }
 };
 
@@ -222,12 +233,12 @@ WalkVariant plan_variant(const mcdp_propagator &P, bool injected);
 size_t plan_lds_bytes(const mcdp_propagator &P, WalkVariant v);
 // The host-buffer entry points' device workspace of at least `need` bytes and
 // stream on the current device (made or grown on demand).  The caller holds
-// P.host_mu until its work on the stream is done, and ends by waiting on it.
-int host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_t &stream);
-// Frees the current device's workspace if it is larger than
-// kHostWorkKeepBytes (a large call does not pin its buffers for good); the
-// caller holds P.host_mu and its stream is idle.
+// P.host_mu until its work on the stream is done, and ends by waiting on it
+// and calling host_workspace_trim.  Up to kHostWorkKeepBytes the workspace is
+// the propagator's own; a larger one comes from a pool of the process and goes
+// back to it (see LargePool in mcdp_host.cpp).
 constexpr size_t kHostWorkKeepBytes = (size_t)4 << 30;
+int host_workspace(mcdp_propagator &P, size_t need, void *&buf, hipStream_t &stream);
 void host_workspace_trim(mcdp_propagator &P);
 // mcdp_reverse_device with its workspace given: `work` of `work_bytes` bytes,
 // split into as many launches as it needs, and nothing allocated (the

@@ -534,7 +534,7 @@ int mcdp_server_create(int64_t memory_budget, int64_t request_cap, int32_t max_r
         return fail(MCDP_E_DEVICE, "no HIP device available: serving runs on the GPU only");
     auto srv = std::make_unique<mcdp_server>();
     HIP_TRY(hipGetDevice(&srv->device), "hipGetDevice");
-    hipError_t e = hipMalloc(&srv->pool_base, (size_t)memory_budget);
+    hipError_t e = device_malloc(&srv->pool_base, (size_t)memory_budget);
     if (e != hipSuccess)
         return fail(MCDP_E_NOMEM, "hipMalloc (serving pool of " + std::to_string(memory_budget) +
                                       " bytes): " + hipGetErrorString(e));
@@ -596,7 +596,7 @@ int mcdp_server_add_context(mcdp_server *srv, mcdp_propagator *prop, int32_t *ct
             pairs[2 * e] = lo[e];
             pairs[2 * e + 1] = hi[e];
         }
-        hipError_t e = hipMalloc(&d_ranges, pairs.size() * 8);
+        hipError_t e = device_malloc((void **)&d_ranges, pairs.size() * 8);
         if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (event bounds): ") + hipGetErrorString(e));
         e = hipMemcpy(d_ranges, pairs.data(), pairs.size() * 8, hipMemcpyHostToDevice);
         if (e != hipSuccess) {

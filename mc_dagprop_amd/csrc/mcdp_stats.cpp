@@ -55,7 +55,7 @@ int ensure_topo(const mcdp_propagator &P, DeviceCopy &d) {
     off[(size_t)P.E] = (int32_t)np;
     const size_t bytes = sizeof(int32_t) * (off.size() + key.size() + pos.size() + nkey.size() + first.size());
     void *blob = nullptr;
-    hipError_t e = hipMalloc(&blob, std::max<size_t>(bytes, 4));
+    hipError_t e = device_malloc(&blob, std::max<size_t>(bytes, 4));
     if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (predecessor table): ") + hipGetErrorString(e));
     auto *p = static_cast<int32_t *>(blob);
     int32_t *d_off = p, *d_key = d_off + off.size(), *d_pos = d_key + key.size(), *d_nkey = d_pos + pos.size();
