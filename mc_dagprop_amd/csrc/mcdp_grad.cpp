@@ -613,9 +613,11 @@ int mcdp_gradient_host(mcdp_propagator *prop, const int32_t *seeds, int64_t n, c
             rc = hip_fail(e, "hipMemcpy");
             break;
         }
-        rc = mcdp_run_many_device(prop, d_seeds, nc, nc, d_real, d_dur, d_cause, st);
+        // rows of whole 128-byte lines (chunk is a multiple of 16 samples)
+        const int64_t ld = (nc + 15) / 16 * 16;
+        rc = mcdp_run_many_device(prop, d_seeds, nc, ld, d_real, d_dur, d_cause, st);
         if (!rc)
-            rc = mcdp_reverse_device(prop, d_seeds, d_w, d_real, d_dur, d_cause, nc, nc, c0 > 0, d_obj, d_gd, d_ge,
+            rc = mcdp_reverse_device(prop, d_seeds, d_w, d_real, d_dur, d_cause, nc, ld, c0 > 0, d_obj, d_gd, d_ge,
                                      st);
         // the next chunk's seeds overwrite this chunk's (the copy is asynchronous for pageable memory)
         if (!rc && (e = hipStreamSynchronize(st)) != hipSuccess) rc = hip_fail(e, "gradient");

@@ -293,6 +293,9 @@ constexpr int kWideStepCost = 300;
 // groups they were measured to end inside the tiles' time on the network and
 // the small workloads).
 constexpr int64_t kWideMaxGroups = 128;
+// The same where one-sample tiles are the alternative (200 x 100 events, wide
+// steps: 64 groups 1.7 ms, 128 groups 2.3; those tiles: 2.1 for any number).
+constexpr int64_t kWideMaxGroupsHalved = 96;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -1020,7 +1023,7 @@ int level_group(const mcdp_propagator &P, int64_t n, int cus) {
 }
 
 // Whether a run of n samples takes the two-pass route (draw_kernel, then
-// level_kernel) instead of a partial round of the walk: when its estimated time
+// level_kernel; halved: its walk would be of one-sample tiles, see launch) instead of a partial round of the walk: when its estimated time
 // is below a tile's.  The walk's tile costs the same however few of its lanes
 // and of the device's CUs are in use: about 11.5 ns per unit of walk_cost (200 x
 // 100 events, any n up to a round: 3.0 ms; 20 x 10: 88 us), about 15 where
@@ -1032,10 +1035,11 @@ int level_group(const mcdp_propagator &P, int64_t n, int cus) {
 // 12,345 3.3 against 4.8).
 constexpr double kTileSecondsPerCost = 10.5e-9;
 constexpr double kTileSecondsPerCostSpilled = 14e-9;
+constexpr double kHalvedTile = 0.72;            // one-sample tiles (launch), up to 64 samples per CU
 constexpr double kLevelSeconds = 0.45e-6;       // one level of one workgroup
 constexpr double kLevelFixedSeconds = 10e-6;    // the second launch, the tables
 constexpr double kLevelBytesPerSecond = 3.9e12;
-bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus) {
+bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus, bool halved) {
     if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
     build_level_slots(P);
     const int group = level_group(P, n, cus);
@@ -1046,7 +1050,8 @@ bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus) {
     const double moved = (n > per_pass ? padded : (double)n) * (8.0 * P.L + 12.0 * P.E) / kLevelBytesPerSecond;
     const double waves = (n > per_pass ? padded / per_pass : 1.0);
     const double levels = std::max(moved, waves * kLevelSeconds * (double)P.levels.size());
-    const double per_cost = P.n_global > 0 ? kTileSecondsPerCostSpilled : kTileSecondsPerCost;
+    const double per_cost = (P.n_global > 0 ? kTileSecondsPerCostSpilled : kTileSecondsPerCost) *
+                            (halved && n <= (int64_t)cus * kLanes ? kHalvedTile : 1.0);
     return kLevelFixedSeconds + draws + levels < per_cost * (double)P.walk_cost;
 }
 
@@ -1077,10 +1082,11 @@ int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injec
 
 // cause_pos (sampled walks, no cause): the winning entry's position per
 // sample instead of the cause event.  scratch: [L][ld] or null, for a sampled
-// run without a durations output that may take the two-pass route.
+// run without a durations output that may take the two-pass route.  shared:
+// other runs use the device beside this one.
 int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double *dur_in, int64_t n, int64_t ld,
            double *realized, double *durations, int32_t *cause, hipStream_t stream, uint8_t *cause_pos = nullptr,
-           double *scratch = nullptr) {
+           double *scratch = nullptr, bool shared = false) {
     if (n < 0) return fail(MCDP_E_INVALID, "n must be non-negative");
     if (cause_pos && (injected || cause)) return fail(MCDP_E_INVALID, "internal error: positions replace sampled causes");
     if (n > 0 && ld < n) return fail(MCDP_E_INVALID, "ld must be >= n");
@@ -1099,7 +1105,12 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     // durations.  Its plan is uploaded by the first such run: one under
     // stream capture, which can upload nothing, walks unless it is there.
     double *const drawn = durations ? durations : scratch;
-    if (n > 0 && (injected || drawn) && level_route(P, injected, n, cus)) {
+    // whether rows of doubles that the walk writes, or reads durations from,
+    // start on 64-byte sectors
+    const auto on_sector = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 63u) == 0; };
+    const bool sectors = ld % 8 == 0 && on_sector(realized) && on_sector(durations) && on_sector(dur_in);
+    const bool halved_ok = !shared && ((!durations && !injected) || sectors);
+    if (n > 0 && (injected || drawn) && level_route(P, injected, n, cus, halved_ok)) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (!d->level_blob) (void)hipStreamIsCapturing(stream, &capture);
         if (capture == hipStreamCaptureStatusNone) {
@@ -1153,6 +1164,16 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     v1.spl = 1;
     const size_t lds1 = walk_lds_bytes(P, v1);
     int64_t resident1 = 0;
+    // A run of at most one group of 64 samples per CU fits the device in
+    // one-sample tiles at once, which take about seven tenths of a two-sample
+    // tile's time (200 x 100 events, 16,384 samples: 2.13 against 2.95 ms; a
+    // second round of them, from 16,385 samples, 4.2 against 3.6).  They take
+    // more of the device in all, which a run beside others would pay for, and
+    // their 512-byte pieces of rows that do not start on cache sectors cost more
+    // than they save (16,383 samples: 4.3 against 3.2 ms; without durations no
+    // matter).
+    const bool halved =
+        v.spl == 2 && P.tail_mode == 0 && !P.shape_by_caller && halved_ok && n <= (int64_t)cus * kLanes;
     {
         const int64_t full_rounds = ((n + tile - 1) / tile) / resident;
         const int64_t rest = n - full_rounds * resident * tile;
@@ -1160,10 +1181,19 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         if (full_rounds == 0 && rest > 0) {
             // less than one round: the wide steps alone against one round of
             // tiles that hardly fills the device
-            if (P.tail_mode == 2 || (P.tail_mode == 0 && groups <= kWideMaxGroups && P.wide_cost < P.tile_cost)) {
+            if (P.tail_mode == 2 || (P.tail_mode == 0 && groups <= (halved ? kWideMaxGroupsHalved : kWideMaxGroups) &&
+                                     P.wide_cost < P.tile_cost)) {
                 wide = true;
                 n_main = 0;
                 n_tail = n;
+            } else if (halved) {
+                int bpc1 = 0;
+                HIP_TRY(walk_occupancy(v1, P.waves, lds1, &bpc1), "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+                resident1 = (int64_t)cus * bpc1;
+                if (groups <= resident1) {
+                    n_main = 0;
+                    n_tail = n;
+                }
             }
         } else if (full_rounds >= 1 && rest > 0) {
             if (P.tail_mode == 2 ||
@@ -1785,7 +1815,7 @@ int mcdp::short_run(mcdp_propagator &P, bool injected, int64_t n, bool &yes) {
     int device = 0, cus = 0;
     HIP_TRY(hipGetDevice(&device), "hipGetDevice");
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device), "hipDeviceGetAttribute");
-    yes = n > 0 && level_route(P, injected, n, cus);
+    yes = n > 0 && level_route(P, injected, n, cus, true);
     return MCDP_OK;
 }
 
@@ -1813,12 +1843,17 @@ int32_t mcdp::max_entries(const mcdp_propagator &P) {
 }
 
 int mcdp::run_many_positions(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
-                             uint8_t *cause_pos, hipStream_t s, double *scratch) {
+                             uint8_t *cause_pos, hipStream_t s, double *scratch, bool shared) {
     if (!cause_pos) return fail(MCDP_E_INVALID, "positions output is null");
     if (max_entries(P) > kMaxPositionEntries)
         return fail(MCDP_E_INVALID, "winner positions need events of at most 254 predecessor entries");
     if (n > 0 && !seeds_dev) return fail(MCDP_E_INVALID, "seeds is null");
-    return launch(P, false, seeds_dev, nullptr, n, ld, realized, nullptr, nullptr, s, cause_pos, scratch);
+    return launch(P, false, seeds_dev, nullptr, n, ld, realized, nullptr, nullptr, s, cause_pos, scratch, shared);
+}
+
+int mcdp::run_many_shared(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
+                          int32_t *cause, hipStream_t s) {
+    return launch(P, false, seeds_dev, nullptr, n, ld, realized, nullptr, cause, s, nullptr, nullptr, true);
 }
 
 // The range of every duration the sampler can draw for link l, as the device

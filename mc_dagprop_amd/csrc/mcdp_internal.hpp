@@ -310,9 +310,13 @@ Record link_record(const mcdp_propagator &P, int32_t l);
 // asynchronous on s.
 constexpr int32_t kMaxPositionEntries = 254;
 int32_t max_entries(const mcdp_propagator &P);
-// scratch: [L][ld] or null, where short_run asks for it.
+// scratch: [L][ld] or null, where short_run asks for it.  shared: beside other
+// runs (the server's), so the route that occupies least of the device.
 int run_many_positions(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
-                       uint8_t *cause_pos, hipStream_t s, double *scratch = nullptr);
+                       uint8_t *cause_pos, hipStream_t s, double *scratch = nullptr, bool shared = false);
+// run_many without durations beside other runs; asynchronous on s.
+int run_many_shared(mcdp_propagator &P, const int32_t *seeds_dev, int64_t n, int64_t ld, double *realized,
+                    int32_t *cause, hipStream_t s);
 // Bounds that hold for every seed: the durations link l can draw, and every
 // event's realized time (false when an earliest time or max_delay is not
 // finite).

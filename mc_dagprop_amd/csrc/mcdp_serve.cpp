@@ -317,8 +317,8 @@ int launch_request(mcdp_server &srv, Request &r) {
         }
         for (int64_t c0 = 0; c0 < n; c0 += r.chunk) {
             const int64_t m = std::min<int64_t>(r.chunk, n - c0);
-            rc = d_pos ? run_many_positions(*prop, d_seeds + c0, m, r.chunk, d_real, d_pos, s)
-                       : mcdp_run_many_device(prop, d_seeds + c0, m, r.chunk, d_real, nullptr, d_cause, s);
+            rc = d_pos ? run_many_positions(*prop, d_seeds + c0, m, r.chunk, d_real, d_pos, s, nullptr, true)
+                       : run_many_shared(*prop, d_seeds + c0, m, r.chunk, d_real, d_cause, s);
             if (rc) return rc;
             rc = chunk_stats_accumulate(*prop, d_real, d_pos ? nullptr : d_cause, d_pos, (int32_t)m, (int32_t)r.chunk,
                                         c0 == 0, d_st, d_hist, d_cnt, s);
@@ -348,12 +348,12 @@ int launch_request(mcdp_server &srv, Request &r) {
             return MCDP_OK;
         }
     } else if (d_pos) {
-        rc = run_many_positions(*prop, d_seeds, n, n, d_real, d_pos, s);
+        rc = run_many_positions(*prop, d_seeds, n, n, d_real, d_pos, s, nullptr, true);
         if (rc) return rc;
         rc = event_stats_positions(*prop, d_real, d_pos, n, n, (int32_t)nq, r.q.data(), d_mean, nq ? d_quant : nullptr,
                                    d_cnt, s);
     } else {
-        rc = mcdp_run_many_device(prop, d_seeds, n, n, d_real, nullptr, d_cause, s);
+        rc = run_many_shared(*prop, d_seeds, n, n, d_real, d_cause, s);
         if (rc) return rc;
         rc = mcdp_event_stats_device(prop, d_real, d_cause, n, n, (int32_t)nq, r.q.data(), d_mean,
                                      nq ? d_quant : nullptr, d_cnt, s);
@@ -406,7 +406,7 @@ int continue_exact(mcdp_server &srv, Request &r) {
     for (int64_t c0 = 0; c0 < n; c0 += r.chunk) {
         if (c0 == kept) continue;
         const int64_t m = std::min<int64_t>(r.chunk, n - c0);
-        rc = mcdp_run_many_device(prop, r.d_seeds + c0, m, r.chunk, r.d_real, nullptr, nullptr, s);
+        rc = run_many_shared(*prop, r.d_seeds + c0, m, r.chunk, r.d_real, nullptr, s);
         if (rc) return rc;
         rc = exact_stats_pass(*prop, r.d_real, (int32_t)m, (int32_t)r.chunk, r.exact, s);
         if (rc) return rc;

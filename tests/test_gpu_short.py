@@ -125,3 +125,30 @@ def test_signed_zero_caps(gpu, configured: bool) -> None:
     ro, co = oracle.OracleCtx(dag).propagate(dur)
     np.testing.assert_array_equal(bits(r), bits(ro))
     np.testing.assert_array_equal(c, co)
+
+
+@pytest.mark.parametrize("ld_extra", [0, 5])
+@pytest.mark.parametrize("n", [10000, 16384, 16385])
+def test_halved_tiles_match(gpu, n: int, ld_extra: int) -> None:
+    """Up to 64 samples per CU (16,384 on 256) a walk takes one-sample tiles where rows start on sectors: the
+    bits of the configured shape, whole and split."""
+    dag = layered_vectorized(8, 120, 4, network_dists(), 8, 11)
+    ld = n + ld_extra
+    seeds = capi.DeviceBuffer.from_array(np.arange(n, dtype=np.int32))
+    out = []
+    for configured in (False, True):
+        P = capi.Propagator(dag)
+        if configured:
+            P.configure(16, 8, 2)
+        r, d, c = (capi.DeviceBuffer(8 * P.E * ld), capi.DeviceBuffer(8 * P.L * ld), capi.DeviceBuffer(4 * P.E * ld))
+        P.run_many_device(seeds, n, ld, r, d, c)
+        capi.synchronize()
+        res = [r.columns(np.float64, P.E, ld, 0, n), d.columns(np.float64, P.L, ld, 0, n),
+               c.columns(np.int32, P.E, ld, 0, n)]
+        P.run_many_device(seeds, n, ld, r, None, None)
+        capi.synchronize()
+        np.testing.assert_array_equal(bits(r.columns(np.float64, P.E, ld, 0, n)), bits(res[0]))
+        out.append(res)
+    np.testing.assert_array_equal(bits(out[0][0]), bits(out[1][0]))
+    np.testing.assert_array_equal(bits(out[0][1]), bits(out[1][1]))
+    np.testing.assert_array_equal(out[0][2], out[1][2])
