@@ -55,6 +55,43 @@ __device__ __forceinline__ DD dd_add(DD x, DD y) {
 constexpr int kWaves = kBlock / 64;
 static_assert(kWaves == 4, "block reductions merge four waves");
 
+// The value of lane (lane ^ o), by data-parallel moves in the vector unit: a
+// __shfl_xor goes through LDS, and the butterflies of one row are some 80 of
+// them per wave.  o is a power of two below 64; every lane of the wave is
+// active.
+template <typename T>
+__device__ __forceinline__ T xor_lane(T x, int o) {
+    constexpr int kWords = (int)(sizeof(T) / 4);
+    struct Words {
+        uint32_t w[kWords];
+    } u = __builtin_bit_cast(Words, x);
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) {
+        const uint32_t v = u.w[i];
+        if (o == 32) {  // r[0]: the lower half's values in both halves, r[1]: the upper half's
+            const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+            u.w[i] = threadIdx.x & 32 ? r[0] : r[1];
+        } else if (o == 16) {  // the same over the rows of 16 lanes
+            const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+            u.w[i] = threadIdx.x & 16 ? r[0] : r[1];
+        } else if (o == 8) {  // a row turned by 8
+            u.w[i] = __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);
+        } else if (o == 4) {  // lane ^ 7 (half row mirrored), then ^ 3 within the quads
+            u.w[i] = __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+        } else if (o == 2) {
+            u.w[i] = __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
+        } else {
+            u.w[i] = __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
+        }
+    }
+    return __builtin_bit_cast(T, u);
+}
+
+// Lane `from`'s value, `from` the same in every active lane.
+__device__ __forceinline__ uint32_t lane_value(uint32_t x, int from) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, from);
+}
+
 // Butterfly sum over a wave's 64 lanes in a fixed order: the double-double
 // sum and the plain one.  Every step is commutative (TwoSum's error term is
 // exact, so a pair's lanes compute the same double-double), so all lanes end
@@ -62,8 +99,8 @@ static_assert(kWaves == 4, "block reductions merge four waves");
 __device__ __forceinline__ void wave_sum(DD &acc, double &plain) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        acc = dd_add(acc, DD{__shfl_xor(acc.hi, o), __shfl_xor(acc.lo, o)});
-        plain += __shfl_xor(plain, o);
+        acc = dd_add(acc, DD{xor_lane(acc.hi, o), xor_lane(acc.lo, o)});
+        plain += xor_lane(plain, o);
     }
 }
 
@@ -139,7 +176,7 @@ __device__ __forceinline__ void wave_hist_add(uint32_t *hist, bool m, uint32_t d
     const uint64_t mm = __ballot(m);
     if (mm == 0) return;
     const int leader = __ffsll((long long)mm) - 1;
-    const uint32_t d0 = __shfl(digit, leader);
+    const uint32_t d0 = lane_value(digit, leader);
     const uint64_t same = __ballot(m && digit == d0);
     if (lane == leader) atomicAdd(&hist[d0], (uint32_t)__popcll(same));
     if (m && digit != d0) atomicAdd(&hist[digit], 1u);
@@ -173,8 +210,8 @@ __device__ __forceinline__ Extremes merge_extremes(Extremes a, const Extremes &b
 __device__ __forceinline__ Extremes wave_merge_extremes(Extremes x) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        const Extremes y{__shfl_xor(x.mn, o), __shfl_xor(x.mx, o), __shfl_xor(x.cmn, o), __shfl_xor(x.cmx, o),
-                         __shfl_xor(x.nans, o)};
+        const Extremes y{xor_lane(x.mn, o), xor_lane(x.mx, o), xor_lane(x.cmn, o), xor_lane(x.cmx, o),
+                         xor_lane(x.nans, o)};
         x = merge_extremes(x, y);
     }
     return x;
@@ -244,6 +281,8 @@ __device__ __forceinline__ void extremes_pass(const double *__restrict__ row, in
 
 constexpr int kValueBins = kMaxRanks * 256;  // the radix histograms' LDS, reused
 constexpr int kGather = kValueBins / 2;      // keys of one bin gathered into the same LDS
+constexpr int kGatherBins = 8;               // bins gathered together,
+constexpr int kGatherAll = 512;              // and their keys in all
 
 // Rows with ranks outside the masses of their extremes, before any radix
 // pass: one pass counts the row in kValueBins bins of equal width over
@@ -251,10 +290,24 @@ constexpr int kGather = kValueBins / 2;      // keys of one bin gathered into th
 // The bin is monotone in v, so the k-th smallest sample lies in the bin where
 // the running count passes k.  A second pass per distinct bin gathers that
 // bin's keys into LDS (at most kGather), where each rank in it is selected
-// exactly by counting, for every gathered key, the keys below and equal to it.
-// Ranks in bins holding more than kGather keys, and rows whose range is not a
-// positive finite double with a finite bin scale, are left to the radix
-// passes (done[r] stays 0).  Rows with NaNs never get here (every rank done).
+// exactly by counting, for every gathered key, the keys below and equal to it;
+// where the bins are few and small, one pass gathers them all.
+// Ranks in bins holding more than kGather keys that are not all equal, and rows
+// whose range is not a positive finite double with a finite bin scale, are left
+// to the radix passes (done[r] stays 0).  Rows with NaNs never get here (every rank done).
+//
+// Bound by the latency of each row's chain of passes, not by memory: what
+// counts is how few dependent steps a row takes and how many rows are in
+// flight (registers: at 71 a CU holds three workgroups; eight loads in flight
+// per lane took 84 and lost a fifth on rows that end after the first pass, and
+// holding 64 by launch bounds spilled).  The serial parts are spread over the
+// block: a scan over the bins' counts instead of one thread walking 512 sums,
+// one gather for all ranks instead of one per bin, ranks broadcast from lanes
+// instead of read from LDS, butterflies without LDS.  6,000 rows, three
+// quantiles and the mean, normal rows: 1,000 samples 370 -> 136 us, 16,000
+// 725 -> 410, 32,768 1,190 -> 690, 65,536 2,520 -> 1,490; rounded to one
+// decimal 16,000 1,450 -> 1,035; rows at their cap (first pass only) 16,000
+// 158 -> 160, 65,536 520 -> 522 (6.0 TB/s).
 template <int kB>
 __device__ void value_bin_select(const double *__restrict__ row, int32_t n, const Extremes &X, int R, int lane,
                                  uint32_t *vh, uint32_t *seg, uint64_t *prefix, const int32_t *krem, int32_t *done,
@@ -286,30 +339,131 @@ __device__ void value_bin_select(const double *__restrict__ row, int32_t n, cons
     __syncthreads();
     scan([&](double v) { wave_hist_add(vh, true, (uint32_t)bin_of(v), lane); });
     __syncthreads();
+    // The bin of each open rank: thread t holds bins [t per, (t + 1) per), a
+    // scan gives the counts before them, and the thread whose bins hold a rank
+    // finds it among them.
     static_assert(kValueBins % kB == 0, "value bins split evenly over the block");
     constexpr int per = kValueBins / kB;
-    uint32_t t = 0;
-    for (int i = 0; i < per; ++i) t += vh[threadIdx.x * per + i];
-    seg[threadIdx.x] = t;
+    uint32_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) mine += vh[threadIdx.x * per + i];
+    uint32_t upto = mine;  // of the wave's lanes up to this one
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t below = __shfl_up(upto, o);
+        upto += lane >= o ? below : 0;
+    }
+    if (lane == 63) seg[threadIdx.x >> 6] = upto;
     __syncthreads();
-    if ((int)threadIdx.x < R && !done[threadIdx.x]) {
-        const int r = threadIdx.x;
-        int32_t k = krem[r];  // its rank in the row (k < n)
-        int g = 0;
-        while (k >= (int32_t)seg[g]) k -= (int32_t)seg[g++];
-        int b = g * per;
-        while (k >= (int32_t)vh[b]) k -= (int32_t)vh[b++];
+    uint32_t before = upto - mine;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) before += seg[w];
+    // Every wave keeps the ranks in its lanes (lane r: rank r) and broadcasts
+    // them from there: a loop over ranks in LDS would wait for each read.
+    const bool in_r = lane < R;
+    bool open_l = in_r && done[in_r ? lane : 0] == 0;
+    const int32_t krem_l = in_r ? krem[lane] : 0;
+    for (int r = 0; r < R; ++r) {
+        if (!(__ballot(open_l) >> r & 1)) continue;
+        const uint32_t k = (uint32_t)__builtin_amdgcn_readlane(krem_l, r);  // its rank in the row (k < n)
+        if (k < before || k - before >= mine) continue;
+        uint32_t left = k - before;
+        int b = threadIdx.x * per;
+        while (left >= vh[b]) left -= vh[b++];
         vbin[r] = b;
-        vloc[r] = k;
+        vloc[r] = (int32_t)left;
         vcnt[r] = (int32_t)vh[b];
     }
     __syncthreads();
+    const int32_t bin_l = in_r ? vbin[lane] : -1, cnt_l = in_r ? vcnt[lane] : 0, loc_l = in_r ? vloc[lane] : 0;
     uint64_t *cand = reinterpret_cast<uint64_t *>(vh);
+    // The open ranks' distinct bins, at most kGatherBins of them and kGatherAll
+    // keys in all (each key is compared with every other): their keys gathered
+    // in one pass over the row.  A rank's place among them is its place in its
+    // bin behind the gathered bins below.
+    int32_t bins[kGatherBins], nb = 0, total = 0, place_l = loc_l;
+#pragma unroll
+    for (int i = 0; i < kGatherBins; ++i) bins[i] = -1;
     for (int r = 0; r < R; ++r) {
-        if (done[r] || vcnt[r] > kGather) continue;  // uniform (LDS, after a barrier)
-        const int32_t b = vbin[r];
+        const uint64_t same = __ballot(open_l && bin_l == __builtin_amdgcn_readlane(bin_l, r));
+        if (same == 0 || __ffsll((long long)same) - 1 != r) continue;  // done, or a bin met before
+        const int32_t b = __builtin_amdgcn_readlane(bin_l, r), c = __builtin_amdgcn_readlane(cnt_l, r);
+#pragma unroll
+        for (int i = 0; i < kGatherBins; ++i) bins[i] = i == nb ? b : bins[i];
+        place_l += b < bin_l ? c : 0;
+        ++nb;
+        total += c;
+    }
+    // (512 keys are one comparison round of the block, 512 steps; more are
+    // cheaper bin by bin, where a bin of one value needs no comparisons)
+    if (nb <= kGatherBins && total <= kGatherAll) {
         if (threadIdx.x == 0) cand_n = 0;
+        __syncthreads();  // every wave is done with the bins' counts
+        scan([&](double v) {
+            const int32_t b = bin_of(v);
+            bool m = false;
+#pragma unroll
+            for (int i = 0; i < kGatherBins; ++i) m = m || bins[i] == b;
+            if (m) cand[atomicAdd(&cand_n, 1u)] = order_key(v);
+        });
         __syncthreads();
+        const int32_t c = (int32_t)cand_n;  // == total
+        for (int32_t i = threadIdx.x; i < (c + 63) / 64 * 64; i += kB) {  // whole waves, for the broadcasts
+            const uint64_t ki = i < c ? cand[i] : 0;
+            int32_t below = i < c ? 0 : c, same = 0;
+#pragma unroll 4
+            for (int32_t j = 0; j < c; ++j) {
+                const uint64_t kj = cand[j];
+                below += kj < ki ? 1 : 0;
+                same += kj == ki ? 1 : 0;
+            }
+            for (int r = 0; r < R; ++r) {
+                if (!(__ballot(open_l) >> r & 1)) continue;
+                const int32_t k = __builtin_amdgcn_readlane(place_l, r);
+                if (i < c && below <= k && k < below + same) prefix[r] = ki;  // equal keys write the same value
+            }
+        }
+        __syncthreads();
+        if (in_r && threadIdx.x < 64) done[lane] = 1;
+        __syncthreads();
+        return;
+    }
+    // Bin by bin: the keys of one gathered, or, for more than kGather, their
+    // extremes (one value held by many samples fills a bin by itself).
+    for (int r = 0; r < R; ++r) {
+        const int32_t b = __builtin_amdgcn_readlane(bin_l, r);
+        const uint64_t same_bin = __ballot(open_l && bin_l == b);
+        if (same_bin == 0 || !(__ballot(open_l) >> r & 1)) continue;
+        const bool big = __builtin_amdgcn_readlane(cnt_l, r) > kGather;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            cand_n = 0;
+            if (big) {
+                cand[0] = ~0ull;
+                cand[1] = 0;
+            }
+        }
+        __syncthreads();
+        if (big) {
+            uint64_t mn = ~0ull, mx = 0;
+            scan([&](double v) {
+                const uint64_t key = order_key(v);
+                const bool m = bin_of(v) == b;
+                mn = m && key < mn ? key : mn;
+                mx = m && key > mx ? key : mx;
+            });
+            if (mn != ~0ull) {
+                atomicMin((unsigned long long *)&cand[0], (unsigned long long)mn);
+                atomicMax((unsigned long long *)&cand[1], (unsigned long long)mx);
+            }
+            __syncthreads();
+            const bool one = cand[0] == cand[1];
+            if (one && threadIdx.x < 64 && open_l && bin_l == b) {
+                prefix[lane] = cand[0];
+                done[lane] = 1;
+            }
+            open_l = open_l && bin_l != b;  // settled, or left to the radix passes
+            continue;
+        }
         scan([&](double v) {
             const bool m = bin_of(v) == b;
             const uint64_t mm = __ballot(m);
@@ -317,26 +471,34 @@ __device__ void value_bin_select(const double *__restrict__ row, int32_t n, cons
             const int leader = __ffsll((long long)mm) - 1;
             uint32_t base = 0;
             if (lane == leader) base = atomicAdd(&cand_n, (uint32_t)__popcll(mm));
-            base = __shfl(base, leader);
+            base = lane_value(base, leader);
             if (m) cand[base + (uint32_t)__popcll(mm & ((1ull << lane) - 1ull))] = order_key(v);
         });
         __syncthreads();
-        const int32_t c = (int32_t)cand_n;  // == vcnt[r]
-        for (int32_t i = threadIdx.x; i < c; i += kB) {
-            const uint64_t ki = cand[i];
-            int32_t below = 0, same = 0;
-            for (int32_t j = 0; j < c; ++j) {
+        const int32_t c = (int32_t)cand_n;  // == the bin's count
+        int other = 0;  // a tie-heavy row's bin often holds one value only
+        for (int32_t i = threadIdx.x; i < c; i += kB) other |= cand[i] != cand[0] ? 1 : 0;
+        const bool one = __syncthreads_or(other) == 0;
+        for (int32_t i = threadIdx.x; i < (one ? 64 : (c + 63) / 64 * 64); i += kB) {
+            const uint64_t ki = i < c ? cand[i] : 0;
+            int32_t below = i < c ? 0 : c, same = one ? c : 0;
+#pragma unroll 4
+            for (int32_t j = 0; j < (one ? 0 : c); ++j) {
                 const uint64_t kj = cand[j];
                 below += kj < ki ? 1 : 0;
                 same += kj == ki ? 1 : 0;
             }
-            for (int q = 0; q < R; ++q)  // equal keys write the same value
-                if (!done[q] && vbin[q] == b && below <= vloc[q] && vloc[q] < below + same) prefix[q] = ki;
+            for (int q = 0; q < R; ++q) {
+                if (!(same_bin >> q & 1)) continue;
+                const int32_t k = __builtin_amdgcn_readlane(loc_l, q);
+                if (i < c && below <= k && k < below + same) prefix[q] = ki;
+            }
         }
         __syncthreads();
-        if ((int)threadIdx.x < R && !done[threadIdx.x] && vbin[threadIdx.x] == b) done[threadIdx.x] = 1;
-        __syncthreads();
+        if (threadIdx.x < 64 && open_l && bin_l == b) done[lane] = 1;
+        open_l = open_l && bin_l != b;
     }
+    __syncthreads();
 }
 
 // LDS of the quantile kernels' work on one row.
@@ -352,7 +514,7 @@ struct QuantileLds {
     int32_t group_of[kMaxRanks];
     int32_t n_groups;
     int32_t first_pass;
-    uint32_t seg[kQBlock];        // value bins: counts per run of kValueBins / kQBlock bins
+    uint32_t seg[kQWaves];        // value bins: counts of each wave's bins
     int32_t vbin[kMaxRanks];      // per rank: its value bin, rank inside it, the bin's count
     int32_t vloc[kMaxRanks];
     int32_t vcnt[kMaxRanks];
@@ -397,7 +559,7 @@ __device__ __forceinline__ void quantile_row(const double *__restrict__ row, int
             wave_sum(acc, plain);
         } else {
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) plain += __shfl_xor(plain, o);
+            for (int o = 32; o > 0; o >>= 1) plain += xor_lane(plain, o);
         }
         if (lane == 0) {
             ext[threadIdx.x >> 6] = x;
@@ -524,19 +686,18 @@ __device__ __forceinline__ void quantile_row(const double *__restrict__ row, int
                 out[j] = res;
             }
         }
-        __syncthreads();  // prefix[] and ext[] are read above before the next row resets them
     }
 }
 
 // Quantiles of each row; with kMean, also the row means.
 template <bool kMean>
 __global__ void __launch_bounds__(kQBlock) quantile_kernel(const double *__restrict__ realized, int32_t n, uint32_t ld,
-                                                          int32_t E, QuantileArgs qa, double *__restrict__ out,
-                                                          double *__restrict__ mean) {
+                                                            QuantileArgs qa, double *__restrict__ out,
+                                                           double *__restrict__ mean) {
     __shared__ QuantileLds L;
-    for (int32_t e = blockIdx.x; e < E; e += gridDim.x)
-        quantile_row<kMean>(realized + (uint64_t)(uint32_t)e * ld, n, qa, out + (uint64_t)(uint32_t)e * (uint32_t)qa.n_q,
-                            kMean ? mean + e : nullptr, L);
+    const uint32_t e = blockIdx.x;  // one workgroup per row: a loop over rows would hold its invariants in registers
+    quantile_row<kMean>(realized + (uint64_t)e * ld, n, qa, out + (uint64_t)e * (uint32_t)qa.n_q,
+                        kMean ? mean + e : nullptr, L);
 }
 
 // Events with at most this many distinct sources count their row in registers.
@@ -596,7 +757,7 @@ __device__ __forceinline__ void count_row_regs(const int32_t *__restrict__ row, 
     for (int k = 0; k <= NK; ++k) {
         uint32_t t = cnt[k];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+        for (int o = 32; o > 0; o >>= 1) t += xor_lane(t, o);
         if ((threadIdx.x & 63) == 0 && t) atomicAdd(&c_lds[k == 0 ? 0 : 1 + pos[k - 1]], t);
     }
 }
@@ -680,7 +841,7 @@ __device__ __forceinline__ void cause_row(const int32_t *__restrict__ row, int32
                 while (__ballot(pending)) {
                     const uint64_t mm = __ballot(pending);
                     const int leader = __ffsll((long long)mm) - 1;
-                    const int32_t s0 = __shfl(slot, leader);
+                    const int32_t s0 = (int32_t)lane_value((uint32_t)slot, leader);
                     const uint64_t same = __ballot(pending && slot == s0);
                     if ((int)(threadIdx.x & 63) == leader) atomicAdd(&c_lds[s0], (uint32_t)__popcll(same));
                     pending = pending && slot != s0;
@@ -760,7 +921,7 @@ __device__ __forceinline__ void count_pos_regs(const uint8_t *__restrict__ row, 
     for (int k = 0; k <= NP; ++k) {
         uint32_t t = cnt[k];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+        for (int o = 32; o > 0; o >>= 1) t += xor_lane(t, o);
         if ((threadIdx.x & 63) == 0 && t) atomicAdd(&c_lds[k], t);
     }
 }
@@ -796,7 +957,7 @@ __device__ __forceinline__ void cause_pos_row(const uint8_t *__restrict__ row, i
                     while (__ballot(pending)) {
                         const uint64_t mm = __ballot(pending);
                         const int leader = __ffsll((long long)mm) - 1;
-                        const int32_t s0 = __shfl(slot, leader);
+                        const int32_t s0 = (int32_t)lane_value((uint32_t)slot, leader);
                         const uint64_t same = __ballot(pending && slot == s0);
                         if ((int)(threadIdx.x & 63) == leader) atomicAdd(&c_lds[s0], (uint32_t)__popcll(same));
                         pending = pending && slot != s0;
@@ -843,15 +1004,13 @@ __device__ __forceinline__ int32_t find_set(const RowSet *__restrict__ sets, int
     return lo;
 }
 
-__global__ void __launch_bounds__(kQBlock) quantile_sets_kernel(const RowSet *__restrict__ sets, int32_t n_sets,
-                                                                int32_t rows) {
+__global__ void __launch_bounds__(kQBlock) quantile_sets_kernel(const RowSet *__restrict__ sets, int32_t n_sets) {
     __shared__ QuantileLds L;
-    for (int32_t g = blockIdx.x; g < rows; g += gridDim.x) {
-        const RowSet &S = sets[find_set(sets, n_sets, g)];
-        const int32_t e = g - S.row0;
-        quantile_row<true>(S.realized + (uint64_t)(uint32_t)e * S.ld, S.n, S.qa,
-                           S.quant + (uint64_t)(uint32_t)e * (uint32_t)S.qa.n_q, S.mean + e, L);
-    }
+    const int32_t g = blockIdx.x;  // one workgroup per row
+    const RowSet &S = sets[find_set(sets, n_sets, g)];
+    const int32_t e = g - S.row0;
+    quantile_row<true>(S.realized + (uint64_t)(uint32_t)e * S.ld, S.n, S.qa,
+                       S.quant + (uint64_t)(uint32_t)e * (uint32_t)S.qa.n_q, S.mean + e, L);
 }
 
 __global__ void __launch_bounds__(kBlock) mean_sets_kernel(const RowSet *__restrict__ sets, int32_t n_sets,
@@ -1202,7 +1361,7 @@ __global__ void __launch_bounds__(kBlock) exact_pass_kernel(const double *__rest
                         const int leader = __ffsll((long long)mm) - 1;
                         uint32_t base = 0;
                         if (lane == leader) base = atomicAdd(&gt[r].fill, (uint32_t)__popcll(mm));
-                        base = __shfl(base, leader);
+                        base = lane_value(base, leader);
                         const uint32_t pos = base + (uint32_t)__popcll(mm & below);
                         if (mem) {
                             if (pos < t.count)
@@ -1480,7 +1639,7 @@ hipError_t launch_set_stats(const RowSet *sets, int32_t n_sets, int32_t rows, bo
                             hipStream_t stream) {
     if (rows <= 0 || n_sets <= 0) return hipSuccess;
     if (quantiles)
-        hipLaunchKernelGGL(quantile_sets_kernel, dim3((unsigned)rows), dim3(kQBlock), 0, stream, sets, n_sets, rows);
+        hipLaunchKernelGGL(quantile_sets_kernel, dim3((unsigned)rows), dim3(kQBlock), 0, stream, sets, n_sets);
     else
         hipLaunchKernelGGL(mean_sets_kernel, dim3((unsigned)rows), dim3(kBlock), 0, stream, sets, n_sets, rows);
     if (counts) hipLaunchKernelGGL(cause_sets_kernel, dim3((unsigned)rows), dim3(kBlock), 0, stream, sets, n_sets, rows);
@@ -1497,7 +1656,7 @@ hipError_t launch_event_quantiles(const double *realized, int32_t n, int32_t ld,
                                   double *out, double *mean, hipStream_t stream) {
     if (E > 0)
         hipLaunchKernelGGL(mean ? quantile_kernel<true> : quantile_kernel<false>, dim3((unsigned)E), dim3(kQBlock), 0,
-                           stream, realized, n, (uint32_t)ld, E, qa, out, mean);
+                           stream, realized, n, (uint32_t)ld, qa, out, mean);
     return hipGetLastError();
 }
 
