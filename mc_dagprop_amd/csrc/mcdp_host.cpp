@@ -1141,8 +1141,25 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     const size_t lds = walk_lds_bytes(P, v);
     HIP_TRY(walk_occupancy(v, P.waves, lds, &bpc), "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     if (bpc < 1) return fail(MCDP_E_DEVICE, "walk kernel cannot be resident with " + std::to_string(lds) + " bytes of LDS");
+    // Rows that do not start on 64-byte sectors (an odd ld): the pieces that two
+    // tiles write of a sector reach memory as two partial writes, and the walk
+    // falls to about 2.7-3.8 TB/s where whole sectors reach 5.8.  Overlapping
+    // tiles whose stores begin and end on sectors (WalkVariant::shift) compute
+    // one sample in sixteen twice instead.  They are taken where the writes are
+    // the bound: one workgroup per CU, cheap draws for the bytes (kShiftBytesPerCost
+    // of a tile's output per unit of tile_cost; the network and 60 x 100 DAGs with
+    // exponential or gamma laws have about 290, with calibrated laws 195, where the
+    // overlap costs 3-6%), and three quarters of a round or more.  200 x 100, ld = n,
+    // before and after: 17,001 samples 3.7 and 3.2 ms, but 60 x 100 0.95 and 0.98;
+    // 30,001 6.8 and 4.0; 32,767 7.2 and 5.7; 65,537 13.8 and 9.0; 98,303 15.7-19.3
+    // and 13.2.  Not for injected durations (98,303 samples 13.8 and 14.1 ms), of
+    // which most bytes are reads.
+    constexpr double kShiftBytesPerCost = 244.0;
+    v.shift = !injected && durations && !sectors && v.paths == kPathsFast && v.spl == 2 && !v.pos && P.tail_mode == 0 &&
+              bpc == 1 && 4 * n > 3 * (int64_t)cus * kLanes * 2 &&
+              (double)(kLanes * 2) * (8.0 * P.L + 12.0 * P.E) > kShiftBytesPerCost * (double)P.tile_cost;
     const int64_t resident = (int64_t)cus * bpc;
-    const int64_t tile = (int64_t)kLanes * v.spl;
+    const int64_t tile = v.shift ? kShiftStep : (int64_t)kLanes * v.spl;  // samples a tile adds
 
     // A tile's run time hardly depends on how many of its lanes are live, so a
     // last round of only a few tiles costs almost a full round.  The samples
@@ -1162,6 +1179,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     bool wide = false;
     WalkVariant v1 = v;
     v1.spl = 1;
+    v1.shift = false;
     const size_t lds1 = walk_lds_bytes(P, v1);
     int64_t resident1 = 0;
     // A run of at most one group of 64 samples per CU fits the device in
@@ -1213,7 +1231,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         }
     }
     p.n = (int32_t)n_main;
-    p.n_tiles = (int32_t)((n_main + tile - 1) / tile);
+    p.n_tiles = (int32_t)(v.shift ? shifted_tiles(n_main) : (n_main + tile - 1) / tile);
     // The wide steps need no LDS and fewer registers than a tile leaves free
     // on a SIMD, so they run on a second stream beside the tiles, forked from
     // the caller's stream before the tiles and joined after.

@@ -147,7 +147,8 @@ struct SlotRow {
 };
 
 // kPos: the cause output is cause_pos (the winning entry's position), not cause.
-template <bool kInjected, int kPaths, int K, int kSpl, bool kPos = false>
+// kShift: the tile is one of the overlapping ones (see kShiftStep).
+template <bool kInjected, int kPaths, int K, int kSpl, bool kPos = false, bool kShift = false>
 __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, double *lds, const LogTable &lt) {
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -176,7 +177,20 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
     // their stores rewrite its bytes unchanged.  No store needs a lane mask.
     uint32_t at8[kSpl];  // byte of the lane's sample in the tile's part of a row of doubles
     uint32_t seed[kSpl];
-    const int32_t s0 = tile * (kLanes * kSpl);
+    // (not with spilled sources: a lane would read back what a neighbour tile stores)
+    static_assert(!kShift || (!kInjected && kSpl == 2 && kPaths == kPathsFast && !kPos), "shifted: sampled, fast, spl 2");
+    const int32_t s0 = tile * (kShift ? kShiftStep : kLanes * kSpl);
+    const uint32_t first_bits = tile == 0 ? 0u : 7u, last_bits = tile == p.n_tiles - 1 ? 8u : 0u;
+    // stores v as sample i of the lane to the row at `row`; shifted: if the sample is in the row's part of the tile
+    auto put = [&](auto v, auto *row, uint32_t &byte, int i) {
+        if (kShift) {
+            const uint32_t a = (0u - (uint32_t)((uintptr_t)row / sizeof(*row))) & 7u;
+            const bool in = i == 0 ? (uint32_t)lane >= (a & first_bits)
+                                   : (uint32_t)lane < (uint32_t)(kShiftStep - kLanes) + (a | last_bits);
+            if (!in) return;
+        }
+        __builtin_nontemporal_store(v, lane_ptr(row, byte));
+    };
 #pragma unroll
     for (int i = 0; i < kSpl; ++i) {
         const int32_t si = s0 + i * kLanes + lane;
@@ -245,7 +259,7 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
                             const uint64_t row = row_offset(cur.i2, ld);
 #pragma unroll
                             for (int i = 0; i < kSpl; ++i)
-                                __builtin_nontemporal_store(dur[i], lane_ptr(durations + row, at8[i]));
+                                put(dur[i], durations + row, at8[i], i);
                         }
                     }
                     double rs[kSpl];
@@ -287,13 +301,13 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
 #pragma unroll
                     for (int i = 0; i < kSpl; ++i) {
                         const double rr = kPaths != kPathsFast && upper < best[i] ? upper : best[i];
-                        __builtin_nontemporal_store(rr, lane_ptr(realized + row, at8[i]));
+                        put(rr, realized + row, at8[i], i);
                         if (kPos) {
                             uint32_t at = at8[i] >> 3;
-                            if (p.cause_pos) __builtin_nontemporal_store((uint8_t)who[i], lane_ptr(cause_pos + row, at));
+                            if (p.cause_pos) put((uint8_t)who[i], cause_pos + row, at, i);
                         } else if (p.cause) {
                             uint32_t at = at8[i] >> 1;
-                            __builtin_nontemporal_store(who[i], lane_ptr(cause + row, at));
+                            put(who[i], cause + row, at, i);
                         }
                         res[j][i] = rr;
                     }
@@ -324,19 +338,19 @@ __device__ __forceinline__ void walk_tile(const WalkParams &p, int32_t tile, dou
             draw(rec, seed, dur);
             const uint64_t row = row_offset(rec.i2, ld);
 #pragma unroll
-            for (int i = 0; i < kSpl; ++i) __builtin_nontemporal_store(dur[i], lane_ptr(durations + row, at8[i]));
+            for (int i = 0; i < kSpl; ++i) put(dur[i], durations + row, at8[i], i);
         }
     }
 }
 
-template <bool kInjected, int kPaths, int K, int kSpl, bool kPos = false>
+template <bool kInjected, int kPaths, int K, int kSpl, bool kPos = false, bool kShift = false>
 __global__ void __launch_bounds__(kMaxWaves * kLanes) walk_kernel(WalkParams p) {
     extern __shared__ double lds[];
     __shared__ LogTableLds log_lds;
     if (!kInjected) stage_log_table(log_lds);
     stage_alias<kInjected, kPaths, kSpl>(p, lds);  // its barrier also publishes the log table
     for (int32_t tile = blockIdx.x; tile < p.n_tiles; tile += gridDim.x)
-        walk_tile<kInjected, kPaths, K, kSpl, kPos>(p, tile, lds, log_lds.view());
+        walk_tile<kInjected, kPaths, K, kSpl, kPos, kShift>(p, tile, lds, log_lds.view());
 }
 
 // Several plans in one launch: workgroups take (plan, tile) items from a
@@ -783,6 +797,12 @@ const void *walk_symbol(int k, int spl) {
 
 // Winner positions (v.pos) only for sampled walks.
 const void *walk_symbol(WalkVariant v) {
+    if (v.shift) {
+        if (v.injected || v.paths != kPathsFast || v.spl != 2 || v.pos) return nullptr;
+        return v.k == 4   ? (const void *)walk_kernel<false, kPathsFast, 4, 2, false, true>
+               : v.k == 8 ? (const void *)walk_kernel<false, kPathsFast, 8, 2, false, true>
+                          : nullptr;
+    }
     if (v.injected)
         return v.pos ? nullptr
                : v.paths == kPathsFast ? walk_symbol<true, kPathsFast, false>(v.k, v.spl)

@@ -54,7 +54,7 @@ struct WalkParams {
     const double *dur_in;   // injected mode: [L][ld]
     int32_t n;              // samples (< 2^31)
     int32_t ld;             // leading dimension of every per-sample array (< 2^31)
-    int32_t n_tiles;        // ceil(n / (64 spl))
+    int32_t n_tiles;        // ceil(n / (64 spl)); WalkVariant::shift: shifted_tiles(n)
     double *realized;       // [E][ld] (read within the launch when a plan spills slots)
     double *durations;      // [L][ld] or null (sampled mode)
     int32_t *cause;         // [E][ld] or null
@@ -77,7 +77,15 @@ struct WalkVariant {
     int k;          // one of kEventsPerWaveChoices
     int spl;        // samples per lane: one of kSplChoices (spl 2: k <= kMaxEventsPerWaveSpl2)
     bool pos = false;  // sampled walks only: the cause output is WalkParams::cause_pos
+    bool shift = false;  // sampled, fast, spl 2, not pos: tiles overlap, each row's stores begin on a cache sector
 };
+
+// Overlapping tiles of 128 lanes begin every 120 samples (fifteen sectors of
+// doubles): tile k stores a row's samples [120 k + a, 120 (k + 1) + a), where a
+// in 0 .. 7 puts that row's first of them on a sector; the first tile also
+// stores those before, the last one, which reaches n, those after.
+constexpr int kShiftStep = 120;
+constexpr int64_t shifted_tiles(int64_t n) { return n > 128 ? (n - 8 + kShiftStep - 1) / kShiftStep : 1; }
 
 hipError_t launch_walk(const WalkParams &p, WalkVariant v, int grid, size_t lds_bytes, hipStream_t stream);
 hipError_t walk_occupancy(WalkVariant v, int waves, size_t lds_bytes, int *blocks_per_cu);
