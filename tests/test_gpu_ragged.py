@@ -2,15 +2,15 @@
 
 Overlapping tiles store each row from its own first whole sector: every row alignment, base pointers
 off the sectors, and sample counts at the edges of a tile, of a round and of its remainder.  What lies
-between the rows' last sample and ld stays as it was.
+between the rows' last sample and ld, and before the first row, stays as it was.
 """
 
 from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import pytest
-import torch
 
 from mc_dagprop_amd import capi
 from mc_dagprop_amd import workloads as wl
@@ -18,21 +18,38 @@ from mc_dagprop_amd import workloads as wl
 pytestmark = pytest.mark.gpu
 
 ROUND = 256 * 120  # samples of one overlapping tile on each CU
+FILL = 0xB3        # byte of memory that no result has been written to
 
 
 class Rows:
-    """An array of rows with `first` elements before it, filled with a value no result takes."""
+    """A device array of rows with `first` elements before it, every byte FILL."""
 
-    def __init__(self, rows: int, ld: int, dtype: torch.dtype, first: int) -> None:
-        self.all = torch.full((first + rows * ld,), -77, dtype=dtype, device="cuda")
-        self.view = self.all[first:].view(rows, ld)
-        self.ptr = ctypes.c_void_p(self.view.data_ptr())
+    def __init__(self, rows: int, ld: int, dtype, first: int) -> None:
+        self.dtype, self.shape, self.first = np.dtype(dtype), (rows, ld), first
+        self.buf = capi.DeviceBuffer((first + rows * ld) * self.dtype.itemsize)
+        capi.check(capi.lib().mcdp_memset(self.buf.ptr, FILL, self.buf.nbytes))
+        self.ptr = ctypes.c_void_p(self.buf.ptr.value + first * self.dtype.itemsize)
+
+    def bits(self) -> tuple[np.ndarray, np.ndarray]:
+        """(the elements before the rows, the rows), as integers."""
+        kind = np.uint64 if self.dtype.itemsize == 8 else np.uint32
+        a = self.buf.to_array(kind, self.first + self.shape[0] * self.shape[1])
+        return a[: self.first], a[self.first :].reshape(self.shape)
 
 
 @pytest.fixture(scope="module")
 def propagator():
-    dag = wl.layered_vectorized(14, 100, 4, wl.network_dists(), 8, 77000)
-    return capi.Propagator(dag)
+    return capi.Propagator(wl.layered_vectorized(6, 100, 4, wl.network_dists(), 8, 77000))
+
+
+def run(P, seeds: np.ndarray, ld: int, first: int, cause: bool = True) -> list[Rows]:
+    out = [Rows(P.E, ld, np.float64, first), Rows(P.L, ld, np.float64, first)]
+    if cause:
+        out.append(Rows(P.E, ld, np.int32, first))
+    d_seeds = capi.DeviceBuffer.from_array(seeds)
+    P.run_many_device(d_seeds, len(seeds), ld, out[0], out[1], out[2] if cause else None)
+    capi.check(capi.lib().mcdp_stream_synchronize(None))
+    return out
 
 
 @pytest.mark.parametrize(
@@ -41,30 +58,17 @@ def propagator():
      (32_767, 0, 0), (45_002, 1, 5), (2 * ROUND + 8, 5, 7), (2 * ROUND + 5003, 0, 2)],
 )
 def test_ragged_rows_equal_aligned_rows(gpu, propagator, n: int, pad: int, first: int) -> None:
-    P = propagator
-    seeds = Rows(1, n, torch.int32, 0)
-    seeds.view[0] = torch.arange(n, dtype=torch.int32) * 3 + 1
-
-    def run(ld: int, first: int) -> list[Rows]:
-        out = [Rows(P.E, ld, torch.float64, first), Rows(P.L, ld, torch.float64, first), Rows(P.E, ld, torch.int32, first)]
-        P.run_many_device(seeds, n, ld, *out)
-        torch.cuda.synchronize()
-        return out
-
-    want = run((n + 15) // 16 * 16, 0)
-    for got, ref in zip(run(n + pad, first), want):
-        assert torch.equal(got.view[:, :n].contiguous().view(torch.int32), ref.view[:, :n].contiguous().view(torch.int32))
-        assert bool((got.view[:, n:] == -77).all()) and bool((got.all[:first] == -77).all())
+    seeds = np.arange(n, dtype=np.int32) * 3 + 1
+    want = run(propagator, seeds, (n + 15) // 16 * 16, 0)
+    for got, ref in zip(run(propagator, seeds, n + pad, first), want):
+        before, rows = got.bits()
+        fill = np.frombuffer(bytes([FILL] * rows.dtype.itemsize), rows.dtype)[0]
+        np.testing.assert_array_equal(rows[:, :n], ref.bits()[1][:, :n])
+        assert (rows[:, n:] == fill).all() and (before == fill).all()
 
 
 def test_without_causes(gpu, propagator) -> None:
-    P, n = propagator, 33_001
-    seeds = Rows(1, n, torch.int32, 0)
-    seeds.view[0] = torch.arange(n, dtype=torch.int32)
-    one = [Rows(P.E, n, torch.float64, 0), Rows(P.L, n, torch.float64, 0), Rows(P.E, n, torch.int32, 0)]
-    two = [Rows(P.E, n, torch.float64, 0), Rows(P.L, n, torch.float64, 0)]
-    P.run_many_device(seeds, n, n, *one)
-    P.run_many_device(seeds, n, n, *two, None)
-    torch.cuda.synchronize()
-    for a, b in zip(one, two):
-        assert torch.equal(a.all.view(torch.int64), b.all.view(torch.int64))
+    n = 33_001
+    seeds = np.arange(n, dtype=np.int32)
+    for a, b in zip(run(propagator, seeds, n, 0), run(propagator, seeds, n, 0, cause=False)):
+        np.testing.assert_array_equal(a.bits()[1], b.bits()[1])
