@@ -106,12 +106,15 @@ int mcdp_run_many_device(mcdp_propagator *prop, const int32_t *seeds_dev, int64_
 /* Simulator::run_many (_core.cpp:355-361) on host buffers, synchronous.
  * Outputs event-major with ld = n: realized[E*n], durations[L*n], cause[E*n].
  * The device work runs in chunks of samples (about 2 GiB of device buffers,
- * kept by the propagator up to 4 GiB).  Results of 16 MB and more reach the
+ * kept by the propagator up to 4 GiB; larger ones, of host calls that keep
+ * whole results on the device, go to a bounded pool of the process and are
+ * freed with the propagator that used them last).  Results of 16 MB and more reach the
  * outputs through pinned staging buffers, 64 MB per device, created on the
  * first such call and held until the process ends; calls from several threads
- * take turns on them.  A run of at most 1,024 samples on a plan of 32 steps
- * or more replays a graph of its launches, captured when the same sample count
- * comes twice in a row (the propagator keeps one).  Any output may be NULL to
+ * take turns on them.  A run of at most 1,024 samples that walks a plan of 32
+ * steps or more (a short run mostly takes two launches instead) replays a graph
+ * of its launches, captured when the same sample count comes twice in a row
+ * (the propagator keeps one).  Any output may be NULL to
  * skip it. */
 int mcdp_run_many_host(mcdp_propagator *prop, const int32_t *seeds, int64_t n, double *realized,
                        double *durations, int32_t *cause);
