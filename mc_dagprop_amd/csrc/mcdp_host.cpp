@@ -1428,6 +1428,7 @@ void mcdp::host_workspace_trim(mcdp_propagator &P) {
     for (auto &h : P.host_work)
         if (h.device == device && h.large) {
             (void)hipStreamSynchronize(h.stream);
+            h.drop_graph();  // it may have been captured in this workspace
             large_pool().give(device, h.large, h.large_bytes, &P);
             h.large = nullptr;
             h.large_bytes = 0;
@@ -1650,9 +1651,10 @@ constexpr int32_t kGraphMinSteps = 32;
 // kGraphMaxSamples samples whose key (ShortRunKey) matches the previous call's
 // is captured into a graph and launched as one; while the key stays, later
 // calls replay that graph.  Any other call, or a capture that fails, launches
-// directly.  The caller holds P.host_mu.
-int launch_host_chunk(mcdp_propagator &P, HostWork *hw, bool injected, const int32_t *d_seeds, double *d_dur,
-                      int64_t m, int64_t ld, double *d_real, int32_t *d_cause, hipStream_t st) {
+// directly.  `work` is the workspace that holds the buffers.  The caller holds
+// P.host_mu.
+int launch_host_chunk(mcdp_propagator &P, HostWork *hw, const void *work, bool injected, const int32_t *d_seeds,
+                      double *d_dur, int64_t m, int64_t ld, double *d_real, int32_t *d_cause, hipStream_t st) {
     auto direct = [&] {
         return launch(P, injected, d_seeds, d_dur, m, ld, d_real, injected ? nullptr : d_dur, d_cause, st);
     };
@@ -1662,7 +1664,7 @@ int launch_host_chunk(mcdp_propagator &P, HostWork *hw, bool injected, const int
     if (qc) return qc;
     if (two_pass) return direct();
     ShortRunKey key;
-    key.buf = hw->buf;
+    key.buf = work;
     key.n = m;
     key.ld = ld;
     key.injected = injected;
@@ -1780,7 +1782,7 @@ int run_host(mcdp_propagator &P, bool injected, const int32_t *seeds, const doub
             rc = hip_fail(e, "hipMemcpy (inputs)");
             break;
         }
-        rc = launch_host_chunk(P, hw, injected, d_seeds, d_dur, m, chunk, d_real, d_cause, st);
+        rc = launch_host_chunk(P, hw, work, injected, d_seeds, d_dur, m, chunk, d_real, d_cause, st);
         if (rc) break;
         prefault.join();  // the pages are ready before the first copy writes them
         const size_t out_bytes = (size_t)m * ((realized ? 8 * E : 0) + (cause ? 4 * E : 0) +

@@ -1,0 +1,25 @@
+"""What the host code keeps on the device between calls, on the CPU: tests/native/device_state runs the host sources
+against a stand-in for the HIP runtime that knows which memory is allocated, what a stream capture forbids and
+what a captured graph launches."""
+
+from __future__ import annotations
+
+import subprocess
+from pathlib import Path
+
+import pytest
+
+NATIVE = Path(__file__).resolve().parent / "native"
+
+
+@pytest.fixture(scope="module")
+def driver() -> Path:
+    res = subprocess.run(["make", "-C", str(NATIVE), "-j8", "_build/device_state"], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout[-3000:] + res.stderr[-3000:]
+    return NATIVE / "_build" / "device_state"
+
+
+@pytest.mark.parametrize("scenario", ["graph_of_large_workspace"])
+def test_device_state(driver: Path, scenario: str) -> None:
+    res = subprocess.run([str(driver), scenario], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0 and res.stdout.strip() == "OK", res.stdout + res.stderr
