@@ -413,7 +413,11 @@ int mcdp_event_record(void *event, void *stream);
 int mcdp_event_elapsed_ms(void *start, void *stop, float *ms);
 /* Stream capture into a HIP graph: begin on `stream` (global capture mode),
  * end returns an instantiated graph; launch replays it on a stream; destroy
- * frees it. */
+ * frees it.  Device runs of a propagator (mcdp_run_many_device,
+ * mcdp_propagate_device) may be captured once it has run on the device,
+ * whatever the size of that run: a plan that the captured run needs and the
+ * first one did not is uploaded beside the capture.  A capture of a
+ * propagator's very first run fails. */
 int mcdp_graph_capture_begin(void *stream);
 int mcdp_graph_capture_end(void *stream, void **graph_exec);
 int mcdp_graph_launch(void *graph_exec, void *stream);

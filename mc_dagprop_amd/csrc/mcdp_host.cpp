@@ -783,7 +783,63 @@ int device_entry_impl(mcdp_propagator &P, DeviceCopy *&out) {
     return MCDP_OK;
 }
 
-// Device allocation for the parts added to it, and their upload.
+// While one of these lives, its thread may allocate and upload although a
+// stream is being captured (the default capture mode forbids that to every
+// thread).  A propagator's plans are uploaded when a run first takes a route
+// that needs them, so a caller that ran it once, whatever the route, may
+// capture any run that follows.
+class DuringCapture {
+   public:
+    explicit DuringCapture(bool allowed)
+        : allowed_(allowed && hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+    ~DuringCapture() {
+        if (allowed_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    DuringCapture(const DuringCapture &) = delete;
+    DuringCapture &operator=(const DuringCapture &) = delete;
+
+   private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool allowed_;
+};
+// Whether a run or a statistics call has used the propagator on d's device.
+bool in_use(const DeviceCopy &d) { return d.blob || d.level_blob || d.topo || d.rev; }
+
+// The side stream of d's device and its events (made once).
+int ensure_side(DeviceCopy &d) {
+    hipError_t e = hipSuccess;
+    if (!d.side) e = hipStreamCreateWithFlags(&d.side, hipStreamNonBlocking);
+    if (e == hipSuccess && !d.fork) e = hipEventCreateWithFlags(&d.fork, hipEventDisableTiming);
+    if (e == hipSuccess && !d.join) e = hipEventCreateWithFlags(&d.join, hipEventDisableTiming);
+    return e == hipSuccess ? MCDP_OK : hip_fail(e, "side stream");
+}
+
+// A device allocation holding `bytes` of `host`.  For a device in use (see
+// DuringCapture) the copy goes through the side stream, which no capture
+// waits for.
+int upload(DeviceCopy &d, const void *host, size_t bytes, void *&blob) {
+    const bool used = in_use(d);
+    const DuringCapture allow(used);
+    int rc = used ? ensure_side(d) : MCDP_OK;
+    if (rc) return rc;
+    void *p = nullptr;
+    hipError_t e = device_malloc(&p, std::max<size_t>(bytes, 256));
+    if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
+    if (used) {
+        e = hipMemcpyAsync(p, host, bytes, hipMemcpyHostToDevice, d.side);
+        if (e == hipSuccess) e = hipStreamSynchronize(d.side);
+    } else {
+        e = hipMemcpy(p, host, bytes, hipMemcpyHostToDevice);
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return hip_fail(e, "hipMemcpy (plan)");
+    }
+    blob = p;
+    return MCDP_OK;
+}
+
+// Parts of one device allocation.
 class Upload {
    public:
     template <typename T>
@@ -793,18 +849,7 @@ class Upload {
         if (!v.empty()) std::memcpy(host_.data() + o, v.data(), v.size() * sizeof(T));
         return o;
     }
-    int send(void *&blob) {
-        blob = nullptr;
-        hipError_t e = device_malloc(&blob, std::max<size_t>(host_.size(), 256));
-        if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
-        e = hipMemcpy(blob, host_.data(), host_.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            (void)hipFree(blob);
-            blob = nullptr;
-            return hip_fail(e, "hipMemcpy (plan)");
-        }
-        return MCDP_OK;
-    }
+    int send(DeviceCopy &d, void *&blob) { return upload(d, host_.data(), host_.size(), blob); }
 
    private:
     std::vector<unsigned char> host_;
@@ -822,7 +867,7 @@ int ensure_levels(const mcdp_propagator &P, DeviceCopy &d) {
     const size_t o_off = up.add(lv.off), o_quad = up.add(lv.quad), o_xof = up.add(lv.extra_of), o_init = up.add(lv.init),
                  o_extra = up.add(lv.extra), o_draws = up.add(lv.draws), o_dist = up.add(P.dist),
                  o_alias = up.add(P.alias);
-    const int rc = up.send(d.level_blob);
+    const int rc = up.send(d, d.level_blob);
     if (rc) return rc;
     const void *b = d.level_blob;
     d.levels.off = part<int32_t>(b, o_off);
@@ -884,25 +929,14 @@ int ensure_device_impl(mcdp_propagator &P, DeviceCopy *&out) {
     put(o_earl, P.earliest.data(), P.earliest.size() * sizeof(double));
     put(o_evrec, P.ev_rec.data(), P.ev_rec.size() * sizeof(int32_t));
     void *blob = nullptr;
-    hipError_t e = device_malloc(&blob, total);
-    if (e != hipSuccess) return fail(MCDP_E_NOMEM, std::string("hipMalloc (plan): ") + hipGetErrorString(e));
-    e = hipMemcpy(blob, host.data(), total, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(blob);
-        return hip_fail(e, "hipMemcpy (plan)");
-    }
+    const int up = upload(d, host.data(), total, blob);
+    if (up) return up;
     // the side stream of wide steps and its fork / join events, made here so
     // that a launch creates nothing (it may be under stream capture)
-    e = hipStreamCreateWithFlags(&d.side, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&d.fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&d.join, hipEventDisableTiming);
-    if (e != hipSuccess) {
-        if (d.side) (void)hipStreamDestroy(d.side);
-        if (d.fork) (void)hipEventDestroy(d.fork);
-        d.side = nullptr;
-        d.fork = nullptr;
+    const int side = ensure_side(d);
+    if (side) {
         (void)hipFree(blob);
-        return hip_fail(e, "side stream");
+        return side;
     }
     d.blob = blob;
     auto *b = static_cast<unsigned char *>(blob);

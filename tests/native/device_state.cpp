@@ -65,12 +65,95 @@ void graph_of_large_workspace() {
     CHECK(fake::graph_launches > before);  // ten chunks in one workspace still replay a graph
 }
 
+// Device arrays of a run of n samples.
+struct Rows {
+    void *seeds = nullptr, *realized = nullptr, *durations = nullptr, *cause = nullptr;
+    int64_t n;
+    Rows(const Dag &d, int64_t n_) : n(n_) {
+        OK(mcdp_malloc(&seeds, 4 * n));
+        OK(mcdp_malloc(&realized, 8 * n * d.E));
+        OK(mcdp_malloc(&durations, 8 * n * d.L));
+        OK(mcdp_malloc(&cause, 4 * n * d.E));
+    }
+    int run(const Dag &d, bool with_durations, void *stream) const {
+        return mcdp_run_many_device(d.p, (const int32_t *)seeds, n, n, (double *)realized,
+                                    with_durations ? (double *)durations : nullptr, (int32_t *)cause, stream);
+    }
+    ~Rows() {
+        for (void *p : {seeds, realized, durations, cause}) OK(mcdp_free(p));
+    }
+};
+
+// A propagator that has run once, short (two launches) or long (the walk): a
+// run of the other kind is captured and replayed, with nothing allocated by
+// the replay.
+void capture_after_a_run(bool first_short, bool durations, int64_t n) {
+    Dag d(20, 30);
+    const Rows first(d, first_short ? 10 : 200000), then(d, n);
+    void *stream = nullptr, *graph = nullptr;
+    OK(mcdp_stream_create(&stream));
+    OK(first.run(d, true, nullptr));
+    OK(mcdp_graph_capture_begin(stream));
+    OK(then.run(d, durations, stream));
+    OK(mcdp_graph_capture_end(stream, &graph));
+    if (graph) {
+        const int allocated = fake::allocations, launched = fake::launches;
+        OK(mcdp_graph_launch(graph, stream));
+        CHECK(fake::launches > launched && fake::allocations == allocated);
+        OK(mcdp_graph_destroy(graph));
+    }
+    OK(mcdp_stream_destroy(stream));
+}
+
+// A propagator that has only walked runs short beside another stream's
+// capture, which goes on.
+void short_run_beside_a_capture() {
+    Dag d(20, 30), other(20, 30);
+    const Rows walk(d, 200000), small(d, 10), captured(other, 200000);
+    void *stream = nullptr, *beside = nullptr, *graph = nullptr;
+    OK(mcdp_stream_create(&stream));
+    OK(mcdp_stream_create(&beside));
+    OK(walk.run(d, true, nullptr));
+    OK(captured.run(other, true, nullptr));
+    OK(mcdp_graph_capture_begin(stream));
+    OK(captured.run(other, true, stream));
+    OK(small.run(d, true, beside));
+    OK(mcdp_graph_capture_end(stream, &graph));
+    if (graph) OK(mcdp_graph_destroy(graph));
+    OK(mcdp_stream_destroy(stream));
+    OK(mcdp_stream_destroy(beside));
+}
+
+// A propagator that has not run has nothing on the device: a capture of its
+// first run fails, and the propagator works afterwards.
+void capture_of_a_first_run() {
+    Dag d(20, 30);
+    const Rows rows(d, 200000);
+    void *stream = nullptr, *graph = nullptr;
+    OK(mcdp_stream_create(&stream));
+    OK(mcdp_graph_capture_begin(stream));
+    CHECK(rows.run(d, true, stream) != MCDP_OK);
+    CHECK(mcdp_graph_capture_end(stream, &graph) != MCDP_OK);
+    OK(rows.run(d, true, stream));
+    OK(mcdp_stream_destroy(stream));
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "graph_of_large_workspace") {
         graph_of_large_workspace();
+    } else if (what == "capture_of_a_walk_after_a_short_run") {
+        capture_after_a_run(true, true, 200000);
+    } else if (what == "capture_without_durations_after_a_short_run") {
+        capture_after_a_run(true, false, 10);
+    } else if (what == "capture_of_a_short_run_after_a_walk") {
+        capture_after_a_run(false, true, 10);
+    } else if (what == "short_run_beside_a_capture") {
+        short_run_beside_a_capture();
+    } else if (what == "capture_of_a_first_run") {
+        capture_of_a_first_run();
     } else {
         std::printf("no such scenario\n");
         return 1;

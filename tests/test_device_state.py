@@ -19,7 +19,17 @@ def driver() -> Path:
     return NATIVE / "_build" / "device_state"
 
 
-@pytest.mark.parametrize("scenario", ["graph_of_large_workspace"])
+SCENARIOS = [
+    "graph_of_large_workspace",
+    "capture_of_a_walk_after_a_short_run",
+    "capture_without_durations_after_a_short_run",
+    "capture_of_a_short_run_after_a_walk",
+    "short_run_beside_a_capture",
+    "capture_of_a_first_run",
+]
+
+
+@pytest.mark.parametrize("scenario", SCENARIOS)
 def test_device_state(driver: Path, scenario: str) -> None:
     res = subprocess.run([str(driver), scenario], capture_output=True, text=True, timeout=300)
     assert res.returncode == 0 and res.stdout.strip() == "OK", res.stdout + res.stderr
