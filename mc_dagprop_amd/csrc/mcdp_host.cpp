@@ -1149,9 +1149,11 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         if (!d->level_blob) (void)hipStreamIsCapturing(stream, &capture);
         if (capture == hipStreamCaptureStatusNone) {
             rc = ensure_levels(P, *d);
-            return rc ? rc
-                      : launch_level_route(P, *d, injected, seeds, dur_in, n, ld, realized, drawn, cause, cause_pos, cus,
-                                           stream);
+            if (!rc)
+                return launch_level_route(P, *d, injected, seeds, dur_in, n, ld, realized, drawn, cause, cause_pos, cus,
+                                          stream);
+            if (rc != MCDP_E_NOMEM) return rc;
+            (void)hipGetLastError();  // no room for its plan: the walk's may be there
         }
     }
     if (!P.shape_fixed) {  // first walk: fit the schedule to this device

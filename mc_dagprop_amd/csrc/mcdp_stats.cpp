@@ -378,23 +378,27 @@ int mcdp_run_stats_host(mcdp_propagator *prop, const int32_t *seeds, int64_t n, 
     const size_t o_mean = o_cause + 256 * (((size_t)(E * n) * cb + 255) / 256);
     const size_t o_q = o_mean + (size_t)E * 8;
     const size_t o_cnt = o_q + (size_t)E * (size_t)std::max(n_q, 0) * 8;
-    size_t bytes = o_cnt + (size_t)(E + P) * 8;
+    const size_t bytes = o_cnt + (size_t)(E + P) * 8;
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
         return fail(MCDP_E_DEVICE, "no HIP device available: statistics run on the GPU only");
     std::lock_guard<std::mutex> host_lock(prop->host_mu);
-    // a short run draws its durations first, into the workspace
+    // a short run draws its durations first, into the workspace, where there
+    // is room for them
     bool two_pass = false;
     rc = short_run(*prop, false, n, two_pass);
     if (rc) return rc;
     const size_t o_dur = 256 * ((bytes + 255) / 256);
-    // (within what a propagator keeps, so that no call needs memory it can
-    // only have for the faster route)
-    two_pass = two_pass && o_dur + (size_t)prop->L * (size_t)n * 8 <= kHostWorkKeepBytes;
-    if (two_pass) bytes = o_dur + (size_t)prop->L * (size_t)n * 8;
+    const size_t with_dur = o_dur + (size_t)prop->L * (size_t)n * 8;
+    two_pass = two_pass && with_dur <= kHostWorkKeepBytes;  // (what a propagator keeps)
     void *buf = nullptr;
     hipStream_t st = nullptr;
-    rc = host_workspace(*prop, bytes, buf, st);
+    rc = host_workspace(*prop, two_pass ? with_dur : bytes, buf, st);
+    if (rc == MCDP_E_NOMEM && two_pass) {  // the walk needs no durations
+        (void)hipGetLastError();
+        two_pass = false;
+        rc = host_workspace(*prop, bytes, buf, st);
+    }
     if (rc) return rc;
     hipError_t e = hipSuccess;
     auto *b = static_cast<unsigned char *>(buf);

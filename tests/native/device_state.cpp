@@ -138,6 +138,39 @@ void capture_of_a_first_run() {
     OK(mcdp_stream_destroy(stream));
 }
 
+// Statistics of a short run on a device with room for its rows, but not for
+// the durations that the two-pass route would hold beside them.
+void statistics_in_little_memory() {
+    Dag d(20, 30);
+    const int64_t n = 2000, rows = n * d.E * 9;
+    const std::vector<int32_t> seeds(n, 1);
+    std::vector<double> mean(d.E);
+    std::vector<int64_t> counts(d.E + d.L);
+    int32_t two_pass = 0;
+    OK(mcdp_debug_short_run(d.p, 0, n, &two_pass));
+    CHECK(two_pass == 1);
+    fake::memory = rows + (4 << 20);
+    for (int i = 0; i < 2; ++i)
+        OK(mcdp_run_stats_host(d.p, seeds.data(), n, 0, nullptr, mean.data(), nullptr, counts.data()));
+    fake::memory = rows / 2;
+    CHECK(mcdp_run_stats_host(d.p, std::vector<int32_t>(2 * n, 1).data(), 2 * n, 0, nullptr, mean.data(), nullptr,
+                              counts.data()) == MCDP_E_NOMEM);
+}
+
+// A short run of a propagator that has walked, on a device with no room left
+// for another plan.
+void short_run_without_room_for_its_plan() {
+    Dag d(20, 30);
+    const Rows walk(d, 200000), small(d, 10);
+    OK(walk.run(d, true, nullptr));
+    fake::memory = fake::used;
+    OK(small.run(d, true, nullptr));
+    fake::memory += (size_t)1 << 30;
+    const int before = fake::allocations;
+    OK(small.run(d, true, nullptr));
+    CHECK(fake::allocations > before);  // two passes as soon as there is room
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -154,6 +187,10 @@ int main(int argc, char **argv) {
         short_run_beside_a_capture();
     } else if (what == "capture_of_a_first_run") {
         capture_of_a_first_run();
+    } else if (what == "statistics_in_little_memory") {
+        statistics_in_little_memory();
+    } else if (what == "short_run_without_room_for_its_plan") {
+        short_run_without_room_for_its_plan();
     } else {
         std::printf("no such scenario\n");
         return 1;

@@ -26,6 +26,8 @@ SCENARIOS = [
     "capture_of_a_short_run_after_a_walk",
     "short_run_beside_a_capture",
     "capture_of_a_first_run",
+    "statistics_in_little_memory",
+    "short_run_without_room_for_its_plan",
 ]
 
 
