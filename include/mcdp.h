@@ -107,8 +107,9 @@ int mcdp_run_many_device(mcdp_propagator *prop, const int32_t *seeds_dev, int64_
  * Outputs event-major with ld = n: realized[E*n], durations[L*n], cause[E*n].
  * The device work runs in chunks of samples (about 2 GiB of device buffers,
  * kept by the propagator up to 4 GiB; larger ones, of host calls that keep
- * whole results on the device, go to a bounded pool of the process and are
- * freed with the propagator that used them last).  Results of 16 MB and more reach the
+ * whole results on the device, go to a pool of the process of at most an eighth
+ * of the device's memory and are freed with the propagator that used them last,
+ * or by mcdp_release_workspaces).  Results of 16 MB and more reach the
  * outputs through pinned staging buffers, 64 MB per device, created on the
  * first such call and held until the process ends; calls from several threads
  * take turns on them.  A run of at most 1,024 samples that walks a plan of 32
@@ -396,6 +397,11 @@ int mcdp_server_set_exact_quantiles(mcdp_server *srv, int32_t exact);
 int mcdp_device_count(int *count);
 int mcdp_malloc(void **ptr, size_t bytes);
 int mcdp_free(void *ptr);
+/* Frees the workspaces of more than 4 GiB that statistics and gradient calls
+ * have left for the next one (at most an eighth of each device's memory), for a
+ * process whose other allocators need it; this library's own allocations take
+ * them back by themselves.  Workspaces in use stay with their calls. */
+int mcdp_release_workspaces(void);
 int mcdp_memcpy_htod(void *dst_dev, const void *src_host, size_t bytes);
 int mcdp_memcpy_dtoh(void *dst_host, const void *src_dev, size_t bytes);
 int mcdp_memset(void *dst_dev, int value, size_t bytes);

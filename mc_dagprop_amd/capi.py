@@ -60,6 +60,7 @@ _SIGNATURES = {
          C.POINTER(_i32)],
     ),
     "mcdp_device_count": (C.c_int, [C.POINTER(C.c_int)]),
+    "mcdp_release_workspaces": (C.c_int, []),
     "mcdp_malloc": (C.c_int, [C.POINTER(_P), C.c_size_t]),
     "mcdp_free": (C.c_int, [_P]),
     "mcdp_memcpy_htod": (C.c_int, [_P, _P, C.c_size_t]),
@@ -650,3 +651,8 @@ class Timer:
 
 def synchronize(stream=None) -> None:
     check(lib().mcdp_stream_synchronize(stream))
+
+
+def release_workspaces() -> None:
+    """Frees the device workspaces above 4 GiB that statistics and gradient calls have left for the next one."""
+    check(lib().mcdp_release_workspaces())

@@ -1319,8 +1319,9 @@ namespace {
 // memory in all, and only while a quarter of it stays free; the oldest goes
 // first.  A propagator's calls and the next propagator's share them (a call
 // owns its workspace from taking it to giving it back, its stream idle), they
-// are freed with the propagator that used them last, and before any allocation
-// of this library fails.
+// are freed with the propagator that used them last, before any allocation of
+// this library fails, and when the caller asks for it, whose other allocators
+// cannot reach them (mcdp_release_workspaces).
 struct LargePool {
     struct Entry {
         int device;
@@ -1351,43 +1352,42 @@ struct LargePool {
         kept.erase(kept.begin() + (std::ptrdiff_t)best);
         return buf;
     }
-    // Keeps or frees an idle workspace of the current device.
+    // Keeps or frees an idle workspace of the current device.  (What goes is
+    // freed after the lock: hipFree waits for the device.)
     void give(int device, void *buf, size_t bytes, const void *owner) {
-        std::lock_guard<std::mutex> lock(mu);
         const Entry e{device, buf, bytes, owner};
+        std::vector<Entry> gone;
         size_t free_bytes = 0, total = 0;
         if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || bytes > total / 8 || free_bytes < total / 4) {
-            release(e);
-            return;
+            gone.push_back(e);
+        } else {
+            std::lock_guard<std::mutex> lock(mu);
+            size_t sum = bytes;
+            for (const Entry &k : kept) sum += k.device == device ? k.bytes : 0;
+            remove([&](const Entry &k) { return k.device == device && sum > total / 8 && ((sum -= k.bytes), true); }, gone);
+            kept.push_back(e);
         }
-        size_t sum = bytes;
-        for (const Entry &k : kept) sum += k.device == device ? k.bytes : 0;
-        for (size_t i = 0; i < kept.size() && sum > total / 8;) {
-            if (kept[i].device != device) {
-                ++i;
-                continue;
-            }
-            sum -= kept[i].bytes;
-            release(kept[i]);
-            kept.erase(kept.begin() + (std::ptrdiff_t)i);
-        }
-        kept.push_back(e);
+        for (const Entry &k : gone) release(k);
     }
     // Frees every kept workspace that `which` names; whether there was one.
     template <typename F>
     bool drop(F &&which) {
-        std::lock_guard<std::mutex> lock(mu);
-        bool any = false;
-        for (size_t i = 0; i < kept.size();) {
-            if (!which(kept[i])) {
-                ++i;
-                continue;
-            }
-            release(kept[i]);
-            kept.erase(kept.begin() + (std::ptrdiff_t)i);
-            any = true;
+        std::vector<Entry> gone;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            remove(which, gone);
         }
-        return any;
+        for (const Entry &k : gone) release(k);
+        return !gone.empty();
+    }
+
+   private:
+    // Moves the kept workspaces that `which` names, oldest first, to `gone`.
+    template <typename F>
+    void remove(F &&which, std::vector<Entry> &gone) {
+        std::vector<Entry> left;
+        for (const Entry &k : kept) (which(k) ? gone : left).push_back(k);
+        kept.swap(left);
     }
 };
 // (never destroyed: propagators may outlive static objects)
@@ -2429,6 +2429,10 @@ int mcdp_device_count(int *count) {
     *count = 0;
     hipError_t e = hipGetDeviceCount(count);
     if (e != hipSuccess) *count = 0;
+    return MCDP_OK;
+}
+int mcdp_release_workspaces(void) {
+    (void)large_pool().drop([](const LargePool::Entry &) { return true; });
     return MCDP_OK;
 }
 int mcdp_malloc(void **ptr, size_t bytes) {

@@ -171,6 +171,28 @@ void short_run_without_room_for_its_plan() {
     CHECK(fake::allocations > before);  // two passes as soon as there is room
 }
 
+// Statistics with a workspace of more than a propagator keeps leave it to the
+// process, which frees it when asked to; the next call has another one.
+void release_of_workspaces() {
+    Dag d(20, 500);
+    const int64_t n = 60000;  // 5.4 GB of rows
+    const std::vector<int32_t> seeds(n, 1);
+    std::vector<double> mean(d.E);
+    auto stats = [&] {
+        OK(mcdp_run_stats_host(d.p, seeds.data(), n, 0, nullptr, mean.data(), nullptr, nullptr));
+    };
+    stats();
+    const size_t held = fake::used;
+    CHECK(held > (size_t)5 << 30);
+    stats();
+    CHECK(fake::used == held);
+    OK(mcdp_release_workspaces());
+    CHECK(fake::used < (size_t)1 << 30);
+    OK(mcdp_release_workspaces());
+    stats();
+    CHECK(fake::used == held);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -191,6 +213,8 @@ int main(int argc, char **argv) {
         statistics_in_little_memory();
     } else if (what == "short_run_without_room_for_its_plan") {
         short_run_without_room_for_its_plan();
+    } else if (what == "release_of_workspaces") {
+        release_of_workspaces();
     } else {
         std::printf("no such scenario\n");
         return 1;

@@ -28,6 +28,7 @@ SCENARIOS = [
     "capture_of_a_first_run",
     "statistics_in_little_memory",
     "short_run_without_room_for_its_plan",
+    "release_of_workspaces",
 ]
 
 
