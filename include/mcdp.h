@@ -458,6 +458,19 @@ int mcdp_debug_tail_mode(mcdp_propagator *prop, int32_t mode);
  * round of the walk.  Results do not depend on it, and a shape set by
  * mcdp_propagator_configure or a tail mode rules it out. */
 int mcdp_debug_short_run(mcdp_propagator *prop, int32_t injected, int64_t n, int32_t *two_pass);
+/* The two-pass route for a propagator: 0 = where it is estimated to be faster
+ * (the default), 1 = wherever it is possible, 2 = never. */
+int mcdp_debug_two_pass_mode(mcdp_propagator *prop, int32_t mode);
+/* What the propagator's last run launched (of a host call in chunks: the last
+ * chunk), as a sum of MCDP_ROUTE_*; MCDP_ROUTE_GRAPH alone if it replayed a
+ * graph.  Tests ask which of the routes they compare were taken. */
+#define MCDP_ROUTE_TWO_PASS 1
+#define MCDP_ROUTE_TILES 2
+#define MCDP_ROUTE_ONE_SAMPLE_TILES 4
+#define MCDP_ROUTE_OVERLAPPING_TILES 8
+#define MCDP_ROUTE_WIDE_STEPS 16
+#define MCDP_ROUTE_GRAPH 32
+int mcdp_debug_last_route(mcdp_propagator *prop, int32_t *route);
 /* The serving footprint rule, host only: for a request of n samples over a
  * context of n_events events and n_preds predecessor entries (at most
  * max_entries for one event: up to 254, chunks store one-byte winner

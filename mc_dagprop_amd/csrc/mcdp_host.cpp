@@ -1075,9 +1075,10 @@ constexpr double kLevelFixedSeconds = 10e-6;    // the second launch, the tables
 constexpr double kLevelBytesPerSecond = 3.9e12;
 bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus, bool halved) {
     if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
+    if (P.two_pass_mode == 2) return false;
     build_level_slots(P);
     const int group = level_group(P, n, cus);
-    if (group == 0) return false;
+    if (group == 0 || P.two_pass_mode == 1) return group != 0;
     const double per_pass = (double)group * cus;  // samples of one workgroup per CU
     const double padded = std::ceil((double)n / per_pass) * per_pass;
     const double draws = injected ? 0.0 : (double)n * 8.0 * P.L / kLevelBytesPerSecond;
@@ -1149,6 +1150,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         if (!d->level_blob) (void)hipStreamIsCapturing(stream, &capture);
         if (capture == hipStreamCaptureStatusNone) {
             rc = ensure_levels(P, *d);
+            P.last_route = MCDP_ROUTE_TWO_PASS;
             if (!rc)
                 return launch_level_route(P, *d, injected, seeds, dur_in, n, ld, realized, drawn, cause, cause_pos, cus,
                                           stream);
@@ -1164,6 +1166,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     rc = ensure_device_impl(P, d);
     if (rc) return rc;
     if (n == 0 || (P.E == 0 && (injected || P.orph.empty()))) return MCDP_OK;
+    P.last_route = 0;
     WalkParams p = d->base;
     p.seeds = seeds;
     p.dur_in = dur_in;
@@ -1277,8 +1280,10 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         HIP_TRY(hipStreamWaitEvent(d->side, d->fork, 0), "hipStreamWaitEvent");
         tail_stream = d->side;
     }
-    if (n_main > 0)
+    if (n_main > 0) {
+        P.last_route |= v.shift ? MCDP_ROUTE_OVERLAPPING_TILES : v.spl == 1 ? MCDP_ROUTE_ONE_SAMPLE_TILES : MCDP_ROUTE_TILES;
         HIP_TRY(launch_walk(p, v, (int)std::min<int64_t>(p.n_tiles, resident), lds, stream), "walk kernel launch");
+    }
     if (n_tail > 0) {
         WalkParams q = p;
         q.seeds = seeds ? seeds + n_main : nullptr;
@@ -1289,6 +1294,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         q.cause_pos = cause_pos ? cause_pos + n_main : nullptr;
         q.n = (int32_t)n_tail;
         q.n_tiles = (int32_t)((n_tail + kLanes - 1) / kLanes);
+        P.last_route |= wide ? MCDP_ROUTE_WIDE_STEPS : MCDP_ROUTE_ONE_SAMPLE_TILES;
         if (wide) {
             const int32_t groups = q.n_tiles;
             const int32_t W = P.waves;
@@ -1706,10 +1712,15 @@ int launch_host_chunk(mcdp_propagator &P, HostWork *hw, const void *work, bool i
     key.injected = injected;
     key.generation = P.generation.load();
     key.tail_mode = P.tail_mode;
-    if (hw->graph && hw->captured == key) {
+    auto replay = [&] {
+        {
+            std::lock_guard<std::mutex> lock(P.mu);
+            P.last_route = MCDP_ROUTE_GRAPH;
+        }
         HIP_TRY(hipGraphLaunch(hw->graph, st), "hipGraphLaunch");
-        return MCDP_OK;
-    }
+        return (int)MCDP_OK;
+    };
+    if (hw->graph && hw->captured == key) return replay();
     if (!(hw->seen == key)) {  // first sight: the shape and the plan's upload happen here, not in a capture
         hw->seen = key;
         return direct();
@@ -1732,8 +1743,7 @@ int launch_host_chunk(mcdp_propagator &P, HostWork *hw, const void *work, bool i
     if (hw->graph) (void)hipGraphExecDestroy(hw->graph);
     hw->graph = exec;
     hw->captured = key;
-    HIP_TRY(hipGraphLaunch(exec, st), "hipGraphLaunch");
-    return MCDP_OK;
+    return replay();
 }
 
 // The host-path state of the current device (after host_workspace).
@@ -2410,6 +2420,21 @@ int mcdp_debug_tail_mode(mcdp_propagator *prop, int32_t mode) {
     if (mode < 0 || mode > 2) return fail(MCDP_E_INVALID, "tail mode must be 0, 1 or 2");
     std::lock_guard<std::mutex> lock(prop->mu);
     prop->tail_mode = mode;
+    return MCDP_OK;
+}
+
+int mcdp_debug_two_pass_mode(mcdp_propagator *prop, int32_t mode) {
+    if (!prop) return fail(MCDP_E_INVALID, "propagator is null");
+    if (mode < 0 || mode > 2) return fail(MCDP_E_INVALID, "two-pass mode must be 0, 1 or 2");
+    std::lock_guard<std::mutex> lock(prop->mu);
+    prop->two_pass_mode = mode;
+    return MCDP_OK;
+}
+
+int mcdp_debug_last_route(mcdp_propagator *prop, int32_t *route) {
+    if (!prop || !route) return fail(MCDP_E_INVALID, "null argument");
+    std::lock_guard<std::mutex> lock(prop->mu);
+    *route = prop->last_route;
     return MCDP_OK;
 }
 

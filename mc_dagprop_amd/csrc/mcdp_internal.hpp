@@ -158,6 +158,8 @@ struct mcdp_propagator {
     // (sum over steps of the costliest event plus the launch gap).
     int64_t tile_cost = 0, wide_cost = 0;
     int32_t tail_mode = 0;  // test hook: 0 by the estimates, 1 tiles, 2 wide steps
+    int32_t two_pass_mode = 0;  // test hook: 0 by the estimate, 1 wherever it can be, 2 never
+    int32_t last_route = 0;     // test hook: MCDP_ROUTE_* of the last run
     int32_t n_steps = 0, waves = 1, slots = 0, max_per_wave = 0, k = mcdp::kMaxEventsPerWave;
     int32_t spl = 1;  // samples per lane of the walk kernel (schedule-independent)
     int64_t n_global = 0;
