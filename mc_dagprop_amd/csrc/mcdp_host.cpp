@@ -293,8 +293,14 @@ constexpr int kWideStepCost = 300;
 // groups they were measured to end inside the tiles' time on the network and
 // the small workloads).
 constexpr int64_t kWideMaxGroups = 128;
-// The same where one-sample tiles are the alternative (200 x 100 events, wide
-// steps: 64 groups 1.7 ms, 128 groups 2.3; those tiles: 2.1 for any number).
+// The same where one-sample tiles, whose time does not depend on the number of
+// groups, are the better alternative above this many: in sampled runs, unless
+// the wide steps cost less than half the tiles or a quarter of the predecessors
+// come from global memory in tiles, which makes those dearer.  Measured with
+// 8,192 samples, wide steps and one-sample tiles: 200 x 100 events 2.33 and 2.07
+// ms (64 groups 1.7); 40 x 60 events of 40 predecessors 1.61 and 2.72; 60 x 250,
+// 37% of the predecessors spilled, 2.34 and 2.99; injected durations, whose tiles
+// are bound by each event's loads: 200 x 100 1.73 and 2.60, 40 x 60 1.06 and 3.29.
 constexpr int64_t kWideMaxGroupsHalved = 96;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -1231,6 +1237,9 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     // matter).
     const bool halved =
         v.spl == 2 && P.tail_mode == 0 && !P.shape_by_caller && halved_ok && n <= (int64_t)cus * kLanes;
+    const bool tiles_early = halved && !injected && 2 * P.wide_cost >= P.tile_cost &&
+                             4 * P.n_global <= (int64_t)P.preds.size();
+    const int64_t wide_max = tiles_early ? kWideMaxGroupsHalved : kWideMaxGroups;
     {
         const int64_t full_rounds = ((n + tile - 1) / tile) / resident;
         const int64_t rest = n - full_rounds * resident * tile;
@@ -1238,8 +1247,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
         if (full_rounds == 0 && rest > 0) {
             // less than one round: the wide steps alone against one round of
             // tiles that hardly fills the device
-            if (P.tail_mode == 2 || (P.tail_mode == 0 && groups <= (halved ? kWideMaxGroupsHalved : kWideMaxGroups) &&
-                                     P.wide_cost < P.tile_cost)) {
+            if (P.tail_mode == 2 || (P.tail_mode == 0 && groups <= wide_max && P.wide_cost < P.tile_cost)) {
                 wide = true;
                 n_main = 0;
                 n_tail = n;

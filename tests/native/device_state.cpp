@@ -20,26 +20,44 @@ int failures = 0;
     } while (0)
 #define OK(call) CHECK((call) == MCDP_OK)
 
-// `layers` x `width` events, one predecessor each (the same place in the layer
-// before), exponential delays.
+// `layers` x `width` events of `preds` predecessors each (the same place in the
+// layer before, and the next ones), exponential delays.
 struct Dag {
     mcdp_propagator *p = nullptr;
     int E, L;
-    Dag(int layers, int width) : E(layers * width), L((layers - 1) * width) {
+    Dag(int layers, int width, int preds = 1) : E(layers * width), L((layers - 1) * width * preds) {
         std::vector<double> earliest(E, 0.0), dur(L, 1.0);
-        std::vector<int32_t> idx(L), type(L, 0), target(L), src(L), act(L);
-        std::vector<int64_t> off(L + 1);
+        std::vector<int32_t> idx(L), type(L, 0), target, src(L), act(L);
+        std::vector<int64_t> off{0};
         for (int l = 0; l < L; ++l) {
-            idx[l] = act[l] = src[l] = l;
-            target[l] = l + width;
-            off[l + 1] = l + 1;
+            const int e = width + l / preds, k = l % preds;
+            idx[l] = act[l] = l;
+            src[l] = (e / width - 1) * width + (e + k) % width;
+            if (k == preds - 1) {
+                target.push_back(e);
+                off.push_back(l + 1);
+            }
         }
         mcdp_generator *gen = nullptr;
         OK(mcdp_generator_create(&gen));
         OK(mcdp_generator_add_exponential(gen, 0, 2.0, 50.0));
-        OK(mcdp_propagator_create(E, earliest.data(), L, idx.data(), dur.data(), type.data(), L, target.data(),
-                                  off.data(), src.data(), act.data(), 1800.0, gen, &p));
+        OK(mcdp_propagator_create(E, earliest.data(), L, idx.data(), dur.data(), type.data(), (int)target.size(),
+                                  target.data(), off.data(), src.data(), act.data(), 1800.0, gen, &p));
         mcdp_generator_destroy(gen);
+    }
+    // what a run of n samples launches
+    int route(int64_t n, bool injected, bool durations, bool two_pass = true) {
+        int32_t r = 0;
+        void *rows = nullptr;
+        OK(mcdp_malloc(&rows, 8));
+        auto *x = (double *)rows;
+        OK(mcdp_debug_two_pass_mode(p, two_pass ? 0 : 2));
+        OK(injected ? mcdp_propagate_device(p, x, n, n, x, (int32_t *)rows, nullptr)
+                    : mcdp_run_many_device(p, (int32_t *)rows, n, n, x, durations ? x : nullptr, (int32_t *)rows, nullptr));
+        OK(mcdp_debug_last_route(p, &r));
+        OK(mcdp_free(rows));
+        fake::dead_accesses = 0;  // (the launchers were given no rows)
+        return r;
     }
     ~Dag() { mcdp_propagator_destroy(p); }
     Dag(const Dag &) = delete;
@@ -193,6 +211,20 @@ void release_of_workspaces() {
     CHECK(fake::used == held);
 }
 
+// Walks of up to 128 groups of 64 samples, where wide steps are the cheaper
+// route although one-sample tiles fit the device at once.
+void wide_steps_below_a_round() {
+    Dag fan(40, 60, 40), net(200, 100, 3), wide(60, 250, 3), light(60, 40, 1);
+    CHECK(fan.route(8000, false, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(fan.route(8192, true, false, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(net.route(6208, true, false, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(net.route(8192, true, false, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(wide.route(8192, false, true, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(light.route(6144, false, false) == MCDP_ROUTE_WIDE_STEPS);
+    CHECK(light.route(8192, false, false) == MCDP_ROUTE_ONE_SAMPLE_TILES);
+    CHECK(net.route(8193, true, false, false) != MCDP_ROUTE_WIDE_STEPS);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -215,6 +247,8 @@ int main(int argc, char **argv) {
         short_run_without_room_for_its_plan();
     } else if (what == "release_of_workspaces") {
         release_of_workspaces();
+    } else if (what == "wide_steps_below_a_round") {
+        wide_steps_below_a_round();
     } else {
         std::printf("no such scenario\n");
         return 1;

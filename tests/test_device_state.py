@@ -29,6 +29,7 @@ SCENARIOS = [
     "statistics_in_little_memory",
     "short_run_without_room_for_its_plan",
     "release_of_workspaces",
+    "wide_steps_below_a_round",
 ]
 
 
