@@ -1010,11 +1010,17 @@ std::vector<Shape> shape_candidates(const mcdp_propagator &P) {
 }
 
 // Picks a shape for the current device without running anything: the most
-// samples resident per CU (workgroups per CU x 64 x samples per lane), then
-// two samples per lane (less scalar work per sample), then the least work on
-// the busiest wave of each step (events x samples per lane, summed over
-// steps), then more waves.  Candidate schedules are built on the host; P is
-// left with the winner.
+// samples resident per CU (workgroups per CU x 64 x samples per lane), those of
+// two-sample lanes counted one and a half times, because a one-sample tile takes
+// 0.72 of a two-sample tile's instructions; then two samples per lane; then the
+// least work on the busiest wave of each step (events x samples per lane,
+// summed over steps), then more waves.  Counted alike, three workgroups of 8
+// waves x 12 events x 1 sample went before one of 16 x 8 x 2 for levels of 65 to 96
+// events: 75 x 80 events, network laws, 65,536 samples 2.75 ms against 2.26,
+// constants without durations 1.38 against 0.92, truncated laws 4.4 against 3.8
+// (131,072: 7.3 and 7.4); and six of 4 x 12 x 1 before two of 8 x 8 x 2 for 33 to
+// 48: 150 x 40 events 2.54 against 2.27, truncated laws 4.05 against 3.74.
+// Candidate schedules are built on the host; P is left with the winner.
 int choose_shape(mcdp_propagator &P) {
     Shape best{P.waves, P.k, 1};
     int64_t best_res = -1, best_load = 0;
@@ -1025,7 +1031,7 @@ int choose_shape(mcdp_propagator &P) {
         const WalkVariant v = walk_variant(P, false);
         int bpc = 0;
         if (walk_occupancy(v, P.waves, walk_lds_bytes(P, v), &bpc) != hipSuccess || bpc < 1) continue;
-        const int64_t res = (int64_t)bpc * kLanes * c.spl;
+        const int64_t res = (int64_t)bpc * kLanes * (c.spl == 2 ? 3 : 1);
         int64_t load = 0;
         for (int32_t t = 0; t < P.n_steps; ++t) {
             int32_t m = 0;

@@ -225,6 +225,19 @@ void wide_steps_below_a_round() {
     CHECK(net.route(8193, true, false, false) != MCDP_ROUTE_WIDE_STEPS);
 }
 
+// The shape a first walk chooses: two samples per lane wherever a step holds the
+// widest level, although one-sample shapes may have more samples resident.
+void shapes_of_two_samples_per_lane() {
+    for (int width : {10, 30, 40, 60, 66, 80, 96, 100, 128}) {
+        Dag d(6, width, 2);
+        int64_t info[10] = {};
+        (void)d.route(200000, false, true);
+        OK(mcdp_propagator_plan_info(d.p, info, 10));
+        if (info[9] != 2) std::printf("width %d: waves %d, events per wave %d\n", width, (int)info[1], (int)info[8]);
+        CHECK(info[0] == 6 && info[9] == 2);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -249,6 +262,8 @@ int main(int argc, char **argv) {
         release_of_workspaces();
     } else if (what == "wide_steps_below_a_round") {
         wide_steps_below_a_round();
+    } else if (what == "shapes_of_two_samples_per_lane") {
+        shapes_of_two_samples_per_lane();
     } else {
         std::printf("no such scenario\n");
         return 1;

@@ -218,8 +218,9 @@ static std::vector<const void *> arrays(const WalkParams &p) {
     return {p.recs, p.seeds, p.dur_in, p.realized, p.durations, p.cause, p.cause_pos};
 }
 hipError_t launch_walk(const WalkParams &p, WalkVariant, int, size_t, hipStream_t s) { return kernel(s, arrays(p)); }
-hipError_t walk_occupancy(WalkVariant, int waves, size_t lds, int *blocks) {
-    *blocks = std::min(16 / waves, (int)((size_t)160 * 1024 / std::max<size_t>(lds, 1)));  // four waves a SIMD
+// As the kernels' registers allow: six waves a SIMD of one sample per lane, four of two.
+hipError_t walk_occupancy(WalkVariant v, int waves, size_t lds, int *blocks) {
+    *blocks = std::min((v.spl == 1 ? 6 : 4) / ((waves + 3) / 4), (int)((size_t)160 * 1024 / std::max<size_t>(lds, 1)));
     return hipSuccess;
 }
 hipError_t launch_walk_wide(const WalkParams &p, bool, int32_t, int32_t, int32_t, hipStream_t s) {

@@ -30,6 +30,7 @@ SCENARIOS = [
     "short_run_without_room_for_its_plan",
     "release_of_workspaces",
     "wide_steps_below_a_round",
+    "shapes_of_two_samples_per_lane",
 ]
 
 
