@@ -505,6 +505,18 @@ int build_schedule(mcdp_propagator &P, int32_t W, int32_t K) {
     return MCDP_OK;
 }
 
+// Threads of a level_kernel workgroup of `group` samples for a widest level of
+// `width` events.
+int level_threads(int32_t width, int group) {
+    const int64_t want = (int64_t)width * group;
+    return (int)std::min<int64_t>((want + kLanes - 1) / kLanes * kLanes, kLevelMaxThreads);
+}
+
+// Microseconds of a level in level_kernel (see two_pass_us): a pass of the
+// workgroup over its items, each of its waves, and in a level with predecessors
+// past the items' inline ones these, one after another.
+constexpr double kLevelPassUs = 0.40, kLevelWaveUs = 0.045, kLevelExtraUs = 0.5, kLevelExtraEachUs = 0.20;
+
 // LDS slots of the two-pass route: an event that a later level reads has one
 // from its own level to the last that reads it.  level_kernel writes a level's
 // results while other waves may still read for that level, so a slot is given
@@ -516,17 +528,38 @@ void build_level_slots(mcdp_propagator &P) {
     const int32_t n_levels = (int32_t)P.levels.size();
     std::vector<int32_t> level((size_t)P.E, 0), last_use((size_t)P.E, -1);
     P.level_width = 0;
-    P.walk_cost = 0;
+    P.walk_cost = P.move_cost = P.level_extra = 0;
+    std::vector<int64_t> extra((size_t)n_levels, 0);  // the most of an event of the level
     for (int32_t t = 0; t < n_levels; ++t) {
         P.level_width = std::max<int32_t>(P.level_width, (int32_t)P.levels[(size_t)t].size());
-        int64_t sum = 0, costliest = 0;
+        int64_t sum = 0, costliest = 0, moves = 0, most = 0;
         for (int32_t e : P.levels[(size_t)t]) {
             level[(size_t)e] = t;
             const int64_t c = event_cost(P, e);
             sum += c;
             costliest = std::max(costliest, c);
+            const int64_t preds = P.pred_off[(size_t)e + 1] - P.pred_off[(size_t)e];
+            const int64_t m = kEventCost + kPredCost * preds;
+            moves += m;
+            most = std::max(most, m);
+            extra[(size_t)t] = std::max(extra[(size_t)t], preds - kLevelPreds);
         }
         P.walk_cost += std::max(costliest, (sum + kMaxWaves - 1) / kMaxWaves);
+        P.move_cost += std::max(most, (moves + kMaxWaves - 1) / kMaxWaves);
+        P.level_extra += extra[(size_t)t];
+    }
+    P.draw_sum = 0;
+    for (int32_t l = 0; l < P.L; ++l)
+        P.draw_sum += draw_cost(P.ldist[(size_t)l] != kNoDistIndex ? &P.dist[P.ldist[(size_t)l]] : nullptr);
+    for (int g = 0; g < 7; ++g) {
+        const int threads = level_threads(P.level_width, 1 << g);
+        const int64_t items = threads >> g;  // of one pass
+        P.level_us[g] = 0.0;
+        for (int32_t t = 0; t < n_levels; ++t) {
+            const int64_t passes = ((int64_t)P.levels[(size_t)t].size() + items - 1) / items, x = extra[(size_t)t];
+            P.level_us[g] += (double)passes * (kLevelPassUs + kLevelWaveUs * (threads / kLanes) +
+                                               (x > 0 ? kLevelExtraUs + kLevelExtraEachUs * (double)x : 0.0));
+        }
     }
     for (int32_t e = 0; e < P.E; ++e)
         for (int64_t k = P.pred_off[(size_t)e]; k < P.pred_off[(size_t)e + 1]; ++k) {
@@ -1068,38 +1101,88 @@ int level_group(const mcdp_propagator &P, int64_t n, int cus) {
     return group;
 }
 
+// Whether a walk of less than a round in one-sample tiles (see launch) takes
+// them rather than wide steps above kWideMaxGroupsHalved groups.
+bool tiles_early(const mcdp_propagator &P, bool injected) {
+    return !injected && 2 * P.wide_cost >= P.tile_cost && 4 * P.n_global <= (int64_t)P.preds.size();
+}
+
+// Estimated microseconds of a walk of n samples, at most a round of tiles; one_sample:
+// in tiles of one sample per lane (see launch).  Wide steps cost a launch gap
+// and their draws or bytes.  A tile's time is its waves' instructions, draws at
+// 4.1 ns a cost unit and the rest at 8.9 (three times that where predecessors
+// come from global memory); with injected durations, which an event waits for,
+// 24 ns a unit of the rest; and some of its bytes.  The plan's costs are those
+// of the shape in use, or of 16 waves while no walk has chosen one.
+double walk_us(const mcdp_propagator &P, bool injected, int64_t n, bool one_sample) {
+    const double bytes = (double)n * (8.0 * (double)P.preds.size() + 12.0 * P.E);
+    const int64_t groups = (n + kLanes - 1) / kLanes;
+    if (groups <= (one_sample && tiles_early(P, injected) ? kWideMaxGroupsHalved : kWideMaxGroups) &&
+        P.wide_cost < P.tile_cost)
+        return injected ? 4.1 * P.n_steps + (bytes + (double)n * 8.0 * (double)P.preds.size()) / 10.2e6 + 0.16 * (double)P.level_extra
+                        : 11.0 + 4.8 * P.n_steps + (double)n * (double)P.draw_sum * 0.047e-6 + 0.27 * (double)P.level_extra;
+    const double shape = P.shape_fixed ? (double)P.tile_cost / (double)std::max<int64_t>(P.walk_cost, 1) : 1.0;
+    const double moves = shape * (double)P.move_cost, draws = shape * (double)P.walk_cost - moves;
+    const bool spilled = P.n_global > 0;
+    const double tile = injected ? 0.0236 * moves * (spilled ? 1.24 : 1.0)
+                                 : 0.0041 * draws + 0.0089 * moves * (spilled ? 3.05 : 1.0) + 0.12 * P.n_steps;
+    return 11.0 + tile * (one_sample ? 1.0 : injected ? 1.09 : 1.36) + bytes / (injected ? 12.5e6 : 13.9e6);
+}
+
+// Estimated microseconds of the two passes.  The draws: their instructions on
+// the device's waves or the longest chain of them on one, and the bytes they
+// write.  The levels: their latency, for as many rounds of workgroups as there
+// are, and the bytes they move, in pieces of a row as long as a workgroup's
+// samples.
+double two_pass_us(const mcdp_propagator &P, bool injected, int64_t n, int group, int cus) {
+    double draws = 0.0;
+    if (!injected) {
+        // a wave takes 256 samples of a link, or those of a short run for several links
+        int64_t samples = (n + 255) / 256 * 256, wave_links = (int64_t)P.L * (samples / 256);
+        if (n < kLanes) {
+            samples = 1;
+            while (samples < n) samples *= 2;
+            wave_links = ((int64_t)P.L * samples + kLanes - 1) / kLanes;
+        }
+        const int64_t waves = (int64_t)cus * 24;
+        const double chain = (double)((wave_links + waves - 1) / waves) * (double)P.draw_sum / std::max(P.L, 1) * 0.038;
+        const double issue = (double)samples * (double)P.draw_sum * 0.0188e-6;
+        draws = 4.0 + std::hypot(std::max(chain, issue), (double)n * 8.0 * P.L / 5.56e6);
+    }
+    int g = 0;
+    while ((1 << g) < group) ++g;
+    const int threads = level_threads(P.level_width, group);
+    const size_t lds = (size_t)P.level_slots * (size_t)group * sizeof(double);
+    const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(kLevelMaxThreads / threads, (int64_t)(kLevelLdsMaxBytes / lds)));
+    const int64_t groups = (n + group - 1) / group;
+    const double rounds = (double)((groups + cus * per_cu - 1) / (cus * per_cu));
+    const double beside = std::min((double)per_cu, std::max(1.0, (double)groups / cus)) - 1.0;
+    const double us_per_mb = group <= 2 ? 0.54 : group == 4 ? 0.27 : group <= 16 ? 0.16 : 0.128;
+    return draws + 3.0 + rounds * P.level_us[g] * (1.0 + 0.3 * beside) +
+           (double)n * (8.0 * (double)P.preds.size() + 12.0 * P.E) * 1e-6 * us_per_mb;
+}
+
 // Whether a run of n samples takes the two-pass route (draw_kernel, then
-// level_kernel; halved: its walk would be of one-sample tiles, see launch) instead of a partial round of the walk: when its estimated time
-// is below a tile's.  The walk's tile costs the same however few of its lanes
-// and of the device's CUs are in use: about 11.5 ns per unit of walk_cost (200 x
-// 100 events, any n up to a round: 3.0 ms; 20 x 10: 88 us), about 15 where
-// predecessors spill to global memory (60 x 250: 4.6 ms); the estimate takes a
-// tenth off, so that a run near the line walks.  The two passes move
-// the durations twice, at about 3.9 TB/s where they are bound by that, but at
-// least a level's latency per level (200 x 100, sampled: 1 sample 0.11 ms, 4,001
-// 1.20, 8,192 2.25 against 2.3 with wide steps, 12,345 3.9 against 3.3; 60 x 250:
-// 12,345 3.3 against 4.8).
-constexpr double kTileSecondsPerCost = 10.5e-9;
-constexpr double kTileSecondsPerCostSpilled = 14e-9;
-constexpr double kHalvedTile = 0.72;            // one-sample tiles (launch), up to 64 samples per CU
-constexpr double kLevelSeconds = 0.45e-6;       // one level of one workgroup
-constexpr double kLevelFixedSeconds = 10e-6;    // the second launch, the tables
-constexpr double kLevelBytesPerSecond = 3.9e12;
+// level_kernel) instead of a partial round of the walk (halved: in one-sample
+// tiles if it is of at most 64 samples per CU): where its estimate is a
+// twentieth below the walk's.  Both estimates' constants are fitted to the times
+// of both routes on 34 DAGs (layered ones of 1 to 2,000 events a level, up to 40
+// predecessors, uneven levels, far predecessors, every kind of law) at up to 11
+// sample counts from 100 to 50,000, sampled and injected: 650 pairs, of which
+// the rule leaves 1 more than 5% slower than its other route (1.06 times) and 15
+// walks that two passes would have beaten by more.  A rule on bytes and a latency
+// per level alone left 54, up to 1.96 times slower: 120 uneven levels of up to 400
+// events, far predecessors, 8,000 samples injected 1.34 ms against 0.92; 71 such
+// levels, up to 12 predecessors, 6,000 samples 3.7 against 2.2.
+constexpr double kTwoPassMargin = 1.05;
 bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus, bool halved) {
     if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
     if (P.two_pass_mode == 2) return false;
     build_level_slots(P);
     const int group = level_group(P, n, cus);
     if (group == 0 || P.two_pass_mode == 1) return group != 0;
-    const double per_pass = (double)group * cus;  // samples of one workgroup per CU
-    const double padded = std::ceil((double)n / per_pass) * per_pass;
-    const double draws = injected ? 0.0 : (double)n * 8.0 * P.L / kLevelBytesPerSecond;
-    const double moved = (n > per_pass ? padded : (double)n) * (8.0 * P.L + 12.0 * P.E) / kLevelBytesPerSecond;
-    const double waves = (n > per_pass ? padded / per_pass : 1.0);
-    const double levels = std::max(moved, waves * kLevelSeconds * (double)P.levels.size());
-    const double per_cost = (P.n_global > 0 ? kTileSecondsPerCostSpilled : kTileSecondsPerCost) *
-                            (halved && n <= (int64_t)cus * kLanes ? kHalvedTile : 1.0);
-    return kLevelFixedSeconds + draws + levels < per_cost * (double)P.walk_cost;
+    return kTwoPassMargin * two_pass_us(P, injected, n, group, cus) <
+           walk_us(P, injected, n, halved && n <= (int64_t)cus * kLanes);
 }
 
 int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injected, const int32_t *seeds,
@@ -1121,8 +1204,7 @@ int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injec
     p.cause = cause;
     p.cause_pos = cause_pos;
     const int group = level_group(P, n, cus);
-    const int64_t want = (int64_t)P.level_width * group;
-    const int threads = (int)std::min<int64_t>((want + kLanes - 1) / kLanes * kLanes, kLevelMaxThreads);
+    const int threads = level_threads(P.level_width, group);
     HIP_TRY(launch_levels(p, P.level_zero_edges, group, threads, P.level_slots, stream), "level kernel launch");
     return MCDP_OK;
 }
@@ -1243,9 +1325,7 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     // matter).
     const bool halved =
         v.spl == 2 && P.tail_mode == 0 && !P.shape_by_caller && halved_ok && n <= (int64_t)cus * kLanes;
-    const bool tiles_early = halved && !injected && 2 * P.wide_cost >= P.tile_cost &&
-                             4 * P.n_global <= (int64_t)P.preds.size();
-    const int64_t wide_max = tiles_early ? kWideMaxGroupsHalved : kWideMaxGroups;
+    const int64_t wide_max = halved && tiles_early(P, injected) ? kWideMaxGroupsHalved : kWideMaxGroups;
     {
         const int64_t full_rounds = ((n + tile - 1) / tile) / resident;
         const int64_t rest = n - full_rounds * resident * tile;

@@ -173,6 +173,10 @@ struct mcdp_propagator {
     std::vector<std::pair<int32_t, int32_t>> level_stale;  // (source, its slot), sources ascending
     int32_t level_slots = 0, level_width = 0;
     int64_t walk_cost = 0;  // a tile's walk in draw-cost units, by 16 waves evenly loaded
+    int64_t move_cost = 0;  // its part without the draws
+    int64_t draw_sum = 0;   // all links' draws, in the same units
+    int64_t level_extra = 0;  // predecessors past an item's inline ones: each level's most, summed
+    double level_us[7] = {};  // estimated latency of all levels, by log2 of the samples per workgroup
     bool level_zero_edges = false;  // some predecessor's edge is outside the link table
     std::shared_ptr<mcdp::RevPlan> rev;  // built on the first gradient call
     int64_t rev_max_tiles = 0;           // test hook: tiles per reverse launch (0: default)

@@ -238,6 +238,25 @@ void shapes_of_two_samples_per_lane() {
     }
 }
 
+// Short runs take two passes where those were measured to be faster, and walk
+// where they were not: with predecessors past an item's inline ones, with
+// few samples a workgroup because many values live, with many rounds.
+void two_passes_where_they_are_faster() {
+    Dag small(20, 10, 2), net(200, 100, 3), wide(60, 250, 3), fan(40, 60, 40), levels2000(6, 2000, 3), seven(9, 59, 7);
+    CHECK(small.route(1, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(net.route(1, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(net.route(1000, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(net.route(4001, true, false) == MCDP_ROUTE_TWO_PASS);
+    CHECK(wide.route(12345, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(fan.route(100, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(fan.route(6000, false, true) != MCDP_ROUTE_TWO_PASS);
+    CHECK(fan.route(6000, true, false) != MCDP_ROUTE_TWO_PASS);
+    CHECK(levels2000.route(8000, true, false) != MCDP_ROUTE_TWO_PASS);
+    CHECK(levels2000.route(20000, true, false) != MCDP_ROUTE_TWO_PASS);
+    CHECK(seven.route(22000, true, false) != MCDP_ROUTE_TWO_PASS);
+    CHECK(net.route(20000, false, true) != MCDP_ROUTE_TWO_PASS);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -264,6 +283,8 @@ int main(int argc, char **argv) {
         wide_steps_below_a_round();
     } else if (what == "shapes_of_two_samples_per_lane") {
         shapes_of_two_samples_per_lane();
+    } else if (what == "two_passes_where_they_are_faster") {
+        two_passes_where_they_are_faster();
     } else {
         std::printf("no such scenario\n");
         return 1;

@@ -31,6 +31,7 @@ SCENARIOS = [
     "release_of_workspaces",
     "wide_steps_below_a_round",
     "shapes_of_two_samples_per_lane",
+    "two_passes_where_they_are_faster",
 ]
 
 
