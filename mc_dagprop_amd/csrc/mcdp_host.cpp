@@ -528,7 +528,7 @@ void build_level_slots(mcdp_propagator &P) {
     const int32_t n_levels = (int32_t)P.levels.size();
     std::vector<int32_t> level((size_t)P.E, 0), last_use((size_t)P.E, -1);
     P.level_width = 0;
-    P.walk_cost = P.move_cost = P.level_extra = 0;
+    P.walk_cost = P.move_cost = P.level_extra = P.draw_sum = 0;
     std::vector<int64_t> extra((size_t)n_levels, 0);  // the most of an event of the level
     for (int32_t t = 0; t < n_levels; ++t) {
         P.level_width = std::max<int32_t>(P.level_width, (int32_t)P.levels[(size_t)t].size());
@@ -544,13 +544,11 @@ void build_level_slots(mcdp_propagator &P) {
             most = std::max(most, m);
             extra[(size_t)t] = std::max(extra[(size_t)t], preds - kLevelPreds);
         }
+        P.draw_sum += sum - moves;
         P.walk_cost += std::max(costliest, (sum + kMaxWaves - 1) / kMaxWaves);
         P.move_cost += std::max(most, (moves + kMaxWaves - 1) / kMaxWaves);
         P.level_extra += extra[(size_t)t];
     }
-    P.draw_sum = 0;
-    for (int32_t l = 0; l < P.L; ++l)
-        P.draw_sum += draw_cost(P.ldist[(size_t)l] != kNoDistIndex ? &P.dist[P.ldist[(size_t)l]] : nullptr);
     for (int g = 0; g < 7; ++g) {
         const int threads = level_threads(P.level_width, 1 << g);
         const int64_t items = threads >> g;  // of one pass

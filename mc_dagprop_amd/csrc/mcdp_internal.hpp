@@ -174,7 +174,7 @@ struct mcdp_propagator {
     int32_t level_slots = 0, level_width = 0;
     int64_t walk_cost = 0;  // a tile's walk in draw-cost units, by 16 waves evenly loaded
     int64_t move_cost = 0;  // its part without the draws
-    int64_t draw_sum = 0;   // all links' draws, in the same units
+    int64_t draw_sum = 0;   // all predecessors' draws, in the same units
     int64_t level_extra = 0;  // predecessors past an item's inline ones: each level's most, summed
     double level_us[7] = {};  // estimated latency of all levels, by log2 of the samples per workgroup
     bool level_zero_edges = false;  // some predecessor's edge is outside the link table
