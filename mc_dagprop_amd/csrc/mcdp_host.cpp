@@ -1040,21 +1040,25 @@ std::vector<Shape> shape_candidates(const mcdp_propagator &P) {
     return out;
 }
 
-// Picks a shape for the current device without running anything: the most
-// samples resident per CU (workgroups per CU x 64 x samples per lane), those of
-// two-sample lanes counted one and a half times, because a one-sample tile takes
-// 0.72 of a two-sample tile's instructions; then two samples per lane; then the
-// least work on the busiest wave of each step (events x samples per lane,
-// summed over steps), then more waves.  Counted alike, three workgroups of 8
-// waves x 12 events x 1 sample went before one of 16 x 8 x 2 for levels of 65 to 96
-// events: 75 x 80 events, network laws, 65,536 samples 2.75 ms against 2.26,
-// constants without durations 1.38 against 0.92, truncated laws 4.4 against 3.8
-// (131,072: 7.3 and 7.4); and six of 4 x 12 x 1 before two of 8 x 8 x 2 for 33 to
-// 48: 150 x 40 events 2.54 against 2.27, truncated laws 4.05 against 3.74.
-// Candidate schedules are built on the host; P is left with the winner.
+// Picks a shape for the current device without running anything.  Among shapes
+// of one number of samples per lane: the most workgroups resident per CU, then
+// the least work on the busiest wave of each step (events, summed over steps),
+// then more waves.  Of the two winners the one of two samples per lane, unless the
+// other has more than one and a half times its work in flight (samples of the
+// resident waves that a step gives an event to): a one-sample tile takes 0.72 of
+// a two-sample tile's instructions.  Compared by samples resident, three workgroups of 8 waves x 12 events x 1 sample went before one of
+// 16 x 8 x 2 for levels of 65 to 96 events: 75 x 80 events, network laws, 65,536
+// samples 2.75 ms against 2.26, constants without durations 1.38 against 0.92,
+// truncated laws 4.4 against 3.8 (131,072: 7.3 and 7.4); and six of 4 x 12 x 1 before
+// two of 8 x 8 x 2 for 33 to 48: 150 x 40 events 2.54 against 2.27, truncated laws
+// 4.05 against 3.74.  Candidate schedules are built on the host; P is left with the winner.
 int choose_shape(mcdp_propagator &P) {
-    Shape best{P.waves, P.k, 1};
-    int64_t best_res = -1, best_load = 0;
+    struct Best {
+        Shape shape{0, 0, 0};
+        int bpc = 0;
+        int64_t load = 0;
+        double flight = 0.0;  // waves with an event, on average over the steps
+    } best[2];
     for (const Shape &c : shape_candidates(P)) {
         int rc = build_schedule(P, c.waves, c.k);
         if (rc) return rc;
@@ -1062,27 +1066,25 @@ int choose_shape(mcdp_propagator &P) {
         const WalkVariant v = walk_variant(P, false);
         int bpc = 0;
         if (walk_occupancy(v, P.waves, walk_lds_bytes(P, v), &bpc) != hipSuccess || bpc < 1) continue;
-        const int64_t res = (int64_t)bpc * kLanes * (c.spl == 2 ? 3 : 1);
-        int64_t load = 0;
+        int64_t load = 0, busy = 0;
         for (int32_t t = 0; t < P.n_steps; ++t) {
             int32_t m = 0;
-            for (int32_t w = 0; w < P.waves; ++w)
-                m = std::max(m, P.ev_off[(size_t)t * P.waves + w + 1] - P.ev_off[(size_t)t * P.waves + w]);
-            load += (int64_t)m * c.spl;
+            for (int32_t w = 0; w < P.waves; ++w) {
+                const int32_t events = P.ev_off[(size_t)t * P.waves + w + 1] - P.ev_off[(size_t)t * P.waves + w];
+                m = std::max(m, events);
+                busy += events > 0 ? 1 : 0;
+            }
+            load += m;
         }
-        const bool better =
-            res > best_res ||
-            (res == best_res &&
-             (c.spl > best.spl ||
-              (c.spl == best.spl && (load < best_load || (load == best_load && c.waves > best.waves)))));
-        if (better) {
-            best_res = res;
-            best_load = load;
-            best = c;
-        }
+        Best &b = best[c.spl - 1];
+        if (bpc > b.bpc || (bpc == b.bpc && (load < b.load || (load == b.load && c.waves > b.shape.waves))))
+            b = Best{c, bpc, load, (double)bpc * (double)busy / std::max(P.n_steps, 1)};
     }
-    P.spl = best.spl;
-    return build_schedule(P, best.waves, best.k);
+    Shape shape{P.waves, P.k, 1};
+    if (best[0].bpc > 0) shape = best[0].shape;
+    if (best[1].bpc > 0 && best[0].flight <= 3.0 * best[1].flight) shape = best[1].shape;
+    P.spl = shape.spl;
+    return build_schedule(P, shape.waves, shape.k);
 }
 
 // Samples per workgroup of level_kernel for a run of n: the fewest that leave
