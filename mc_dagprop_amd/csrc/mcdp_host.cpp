@@ -1165,24 +1165,27 @@ double two_pass_us(const mcdp_propagator &P, bool injected, int64_t n, int group
 // Whether a run of n samples takes the two-pass route (draw_kernel, then
 // level_kernel) instead of a partial round of the walk (halved: in one-sample
 // tiles if it is of at most 64 samples per CU): where its estimate is a
-// twentieth below the walk's.  Both estimates' constants are fitted to the times
+// twentieth below the walk's, a fifth above 64 samples per CU, where the walk's
+// estimate is least certain (179 x 8 events, 31,001 samples 0.60 ms against 0.50
+// by a twentieth).  Both estimates' constants are fitted to the times
 // of both routes on 34 DAGs (layered ones of 1 to 2,000 events a level, up to 40
 // predecessors, uneven levels, far predecessors, every kind of law) at up to 11
 // sample counts from 100 to 50,000, sampled and injected: 650 pairs, of which
-// the rule leaves 1 more than 5% slower than its other route (1.06 times) and 15
-// walks that two passes would have beaten by more.  A rule on bytes and a latency
+// the rule leaves none more than 5% slower than its other route and 15 walks
+// that two passes would have beaten by more.  A rule on bytes and a latency
 // per level alone left 54, up to 1.96 times slower: 120 uneven levels of up to 400
 // events, far predecessors, 8,000 samples injected 1.34 ms against 0.92; 71 such
 // levels, up to 12 predecessors, 6,000 samples 3.7 against 2.2.
-constexpr double kTwoPassMargin = 1.05;
+constexpr double kTwoPassMargin = 1.05, kTwoPassMarginFull = 1.2;
 bool level_route(mcdp_propagator &P, bool injected, int64_t n, int cus, bool halved) {
     if (P.tail_mode != 0 || P.shape_by_caller || P.E == 0 || P.L == 0 || n > kLevelMaxSamples) return false;
     if (P.two_pass_mode == 2) return false;
     build_level_slots(P);
     const int group = level_group(P, n, cus);
     if (group == 0 || P.two_pass_mode == 1) return group != 0;
-    return kTwoPassMargin * two_pass_us(P, injected, n, group, cus) <
-           walk_us(P, injected, n, halved && n <= (int64_t)cus * kLanes);
+    const bool full = n > (int64_t)cus * kLanes;
+    return (full ? kTwoPassMarginFull : kTwoPassMargin) * two_pass_us(P, injected, n, group, cus) <
+           walk_us(P, injected, n, halved && !full);
 }
 
 int launch_level_route(const mcdp_propagator &P, const DeviceCopy &d, bool injected, const int32_t *seeds,

@@ -242,7 +242,8 @@ void shapes_of_two_samples_per_lane() {
 // where they were not: with predecessors past an item's inline ones, with
 // few samples a workgroup because many values live, with many rounds.
 void two_passes_where_they_are_faster() {
-    Dag small(20, 10, 2), net(200, 100, 3), wide(60, 250, 3), fan(40, 60, 40), levels2000(6, 2000, 3), seven(9, 59, 7);
+    Dag small(20, 10, 2), net(200, 100, 3), wide(60, 250, 3), fan(40, 60, 40), levels2000(6, 2000, 3), seven(9, 59, 7),
+        narrow(179, 8, 2), tiny(9, 8, 1);
     CHECK(small.route(1, false, true) == MCDP_ROUTE_TWO_PASS);
     CHECK(net.route(1, false, true) == MCDP_ROUTE_TWO_PASS);
     CHECK(net.route(1000, false, true) == MCDP_ROUTE_TWO_PASS);
@@ -255,6 +256,10 @@ void two_passes_where_they_are_faster() {
     CHECK(levels2000.route(20000, true, false) != MCDP_ROUTE_TWO_PASS);
     CHECK(seven.route(22000, true, false) != MCDP_ROUTE_TWO_PASS);
     CHECK(net.route(20000, false, true) != MCDP_ROUTE_TWO_PASS);
+    CHECK(narrow.route(8192, false, true) == MCDP_ROUTE_TWO_PASS);
+    (void)tiny.route(200000, false, true);  // a walk: the shape is chosen
+    CHECK(tiny.route(1000, false, true) == MCDP_ROUTE_TWO_PASS);
+    CHECK(tiny.route(31001, false, true) != MCDP_ROUTE_TWO_PASS);
 }
 
 }  // namespace
