@@ -292,9 +292,10 @@ constexpr int kGatherAll = 512;              // and their keys in all
 // bin's keys into LDS (at most kGather), where each rank in it is selected
 // exactly by counting, for every gathered key, the keys below and equal to it;
 // where the bins are few and small, one pass gathers them all.
-// Ranks in bins holding more than kGather keys that are not all equal, and rows
-// whose range is not a positive finite double with a finite bin scale, are left
-// to the radix passes (done[r] stays 0).  Rows with NaNs never get here (every rank done).
+// In bins holding more than kGather keys one pass settles the ranks in the mass
+// of a frequent value; other ranks there, and rows whose range is not a positive
+// finite double with a finite bin scale, are left to the radix passes (done[r]
+// stays 0).  Rows with NaNs never get here (every rank done).
 //
 // Bound by the latency of each row's chain of passes, not by memory: what
 // counts is how few dependent steps a row takes and how many rows are in
@@ -307,7 +308,10 @@ constexpr int kGatherAll = 512;              // and their keys in all
 // quantiles and the mean, normal rows: 1,000 samples 370 -> 136 us, 16,000
 // 725 -> 410, 32,768 1,190 -> 690, 65,536 2,520 -> 1,490; rounded to one
 // decimal 16,000 1,450 -> 1,035; rows at their cap (first pass only) 16,000
-// 158 -> 160, 65,536 520 -> 522 (6.0 TB/s).
+// 158 -> 160, 65,536 520 -> 522 (6.0 TB/s).  3,000 rows of which 60% of the samples
+// hold one value inside the range, 32,768 samples: 1,520 -> 480 (the bin of such a
+// value holds others too, so a pass that looked whether all its keys are equal
+// went before the radix passes for nothing); rounded to whole numbers 398 -> 400.
 template <int kB>
 __device__ void value_bin_select(const double *__restrict__ row, int32_t n, const Extremes &X, int R, int lane,
                                  uint32_t *vh, uint32_t *seg, uint64_t *prefix, const int32_t *krem, int32_t *done,
@@ -427,8 +431,9 @@ __device__ void value_bin_select(const double *__restrict__ row, int32_t n, cons
         __syncthreads();
         return;
     }
-    // Bin by bin: the keys of one gathered, or, for more than kGather, their
-    // extremes (one value held by many samples fills a bin by itself).
+    // Bin by bin: the keys of one gathered, or, for more than kGather, the row's
+    // samples below and equal to one of them counted (one value held by many
+    // samples fills a bin almost by itself).
     for (int r = 0; r < R; ++r) {
         const int32_t b = __builtin_amdgcn_readlane(bin_l, r);
         const uint64_t same_bin = __ballot(open_l && bin_l == b);
@@ -437,29 +442,32 @@ __device__ void value_bin_select(const double *__restrict__ row, int32_t n, cons
         __syncthreads();
         if (threadIdx.x == 0) {
             cand_n = 0;
-            if (big) {
-                cand[0] = ~0ull;
-                cand[1] = 0;
-            }
+            if (big) cand[1] = cand[2] = 0;
         }
         __syncthreads();
         if (big) {
-            uint64_t mn = ~0ull, mx = 0;
-            scan([&](double v) {
-                const uint64_t key = order_key(v);
-                const bool m = bin_of(v) == b;
-                mn = m && key < mn ? key : mn;
-                mx = m && key > mx ? key : mx;
-            });
-            if (mn != ~0ull) {
-                atomicMin((unsigned long long *)&cand[0], (unsigned long long)mn);
-                atomicMax((unsigned long long *)&cand[1], (unsigned long long)mx);
-            }
+            const double v = row[threadIdx.x];  // (the row has more than kB samples)
+            const bool in = bin_of(v) == b;
+            if (in) cand[0] = order_key(v);  // any of them: most likely a frequent one
             __syncthreads();
-            const bool one = cand[0] == cand[1];
-            if (one && threadIdx.x < 64 && open_l && bin_l == b) {
-                prefix[lane] = cand[0];
-                done[lane] = 1;
+            const uint64_t key0 = cand[0];
+            const uint64_t pivot = (uint64_t)lane_value((uint32_t)(key0 >> 32), 0) << 32 | lane_value((uint32_t)key0, 0);
+            const double value = key_value(pivot);
+            // without another alike the bin holds no such value (and zeros may be of two signs)
+            if (__syncthreads_count(in && v == value) > 1 && value != 0.0) {
+                uint32_t below = 0, same = 0;
+                scan([&](double x) {
+                    below += x < value ? 1u : 0u;
+                    same += x == value ? 1u : 0u;
+                });
+                if (below) atomicAdd((unsigned long long *)&cand[1], (unsigned long long)below);
+                if (same) atomicAdd((unsigned long long *)&cand[2], (unsigned long long)same);
+                __syncthreads();
+                const int32_t first = (int32_t)cand[1], past = first + (int32_t)cand[2];
+                if (threadIdx.x < 64 && open_l && krem_l >= first && krem_l < past) {
+                    prefix[lane] = pivot;
+                    done[lane] = 1;
+                }
             }
             open_l = open_l && bin_l != b;  // settled, or left to the radix passes
             continue;
