@@ -1059,6 +1059,7 @@ int choose_shape(mcdp_propagator &P) {
         int64_t load = 0;
         double flight = 0.0;  // waves with an event, on average over the steps
     } best[2];
+    Shape shape{P.waves, P.k, 1};
     for (const Shape &c : shape_candidates(P)) {
         int rc = build_schedule(P, c.waves, c.k);
         if (rc) return rc;
@@ -1080,7 +1081,6 @@ int choose_shape(mcdp_propagator &P) {
         if (bpc > b.bpc || (bpc == b.bpc && (load < b.load || (load == b.load && c.waves > b.shape.waves))))
             b = Best{c, bpc, load, (double)bpc * (double)busy / std::max(P.n_steps, 1)};
     }
-    Shape shape{P.waves, P.k, 1};
     if (best[0].bpc > 0) shape = best[0].shape;
     if (best[1].bpc > 0 && best[0].flight <= 3.0 * best[1].flight) shape = best[1].shape;
     P.spl = shape.spl;
@@ -1322,8 +1322,9 @@ int launch(mcdp_propagator &P, bool injected, const int32_t *seeds, const double
     // one-sample tiles at once, which take about seven tenths of a two-sample
     // tile's time (200 x 100 events, 16,384 samples: 2.13 against 2.95 ms; a
     // second round of them, from 16,385 samples, 4.2 against 3.6).  They take
-    // more of the device in all, which a run beside others would pay for, and
-    // their 512-byte pieces of rows that do not start on cache sectors cost more
+    // more of the device in all, which a run beside others pays for (12,000 to
+    // 16,384 samples, on two streams at once 1.07-1.28 times the two-sample tiles'
+    // time, on four 0.85-0.94, alone 0.63-0.67), and their 512-byte pieces of rows that do not start on cache sectors cost more
     // than they save (16,383 samples: 4.3 against 3.2 ms; without durations no
     // matter).
     const bool halved =

@@ -24,7 +24,7 @@
 // paths take v_min_f64 of a candidate that has won already, see capped_at).
 //
 // Bound by instruction issue: a wave-activity of the network workload takes
-// about 125 VALU instructions (4.3 cycles each on a SIMD, 2.4 for one- and
+// 107 VALU instructions (4.3 cycles each on a SIMD, 2.4 for one- and
 // two-operand 32-bit ones) for its two samples.  200 x 100 events, 100,000
 // samples: 11.9 ms -> 11.2 with the integer-indexed logarithm, a lane's two
 // draws side by side, output rows addressed by scalar base and lane offset and
@@ -557,8 +557,8 @@ __global__ void __launch_bounds__(kDrawBlock, kDrawBlocksPerCu) draw_kernel(Draw
 // ahead, over the barriers, in a ring of four stages (the step is written out
 // once per position of the ring, so no stage is ever copied).  Bound by a
 // level's latency for few samples (0.45 us per level: loads one step ahead took
-// 1.0), by the durations' and results' bytes for many (16,384 samples of 200 x
-// 100 events: 10.5 GB in 2.7 ms, 3.9 TB/s, against 4.8 for a plain copy).
+// 1.0), by the durations' and results' bytes for many (8,192 samples of 200 x
+// 100 events: 5.2 GB in 1.47 ms, 3.6 TB/s, against 4.8 for a plain copy).
 struct LevelStage {
     LevelQuad q[kLevelQuads];
     double d[kLevelPreds];
